@@ -69,9 +69,10 @@ __device__ __forceinline__ float sqrt_(float x) { return sqrt_rn(x); }
 // projected point by ~0.5 m = 2e-4 of the shell height and flips density thresholds downstream.
 // Every normalised or measured vector here is a ray direction or a difference of positions at metre
 // scale (squared lengths 0 or far above 2^-96, lengths within [2^-125, 2^125]), so the unscaled forms
-// of the correctly rounded square root and reciprocal apply.
-__device__ __forceinline__ V3 normalize3(V3 a) { return a * rcp_rn(sqrt_rn_normal(dot3(a, a))); }
-__device__ __forceinline__ float length3(V3 a) { return sqrt_rn_normal(dot3(a, a)); }
+// of the correctly rounded square root and reciprocal apply, both taken from one v_rsq_f32. length3 of a zero
+// vector is NaN: its callers scale the length and clamp it to [0, 1], which gives the 0 of a zero length.
+__device__ __forceinline__ V3 normalize3(V3 a) { return a * rcp_sqrt_rn(dot3(a, a)); }
+__device__ __forceinline__ float length3(V3 a) { return sqrt_rn_rsq(dot3(a, a)); }
 __device__ __forceinline__ float clampf(float x, float lo, float hi) { return fminf(fmaxf(x, lo), hi); }
 __device__ __forceinline__ float mixf(float x, float y, float a) { return x * (1.0f - a) + y * a; }
 // Filter lerps: one fused multiply-add, a + t (b - a) rounded once. With 8-bit sub-texel weights every
@@ -135,8 +136,9 @@ __device__ __forceinline__ float remapk(float v, float a, float inv_ba, float c,
 // sits behind a branch that whole waves of empty samples skip.
 __device__ __forceinline__ float remapClamped01(float v, float a) {
     if (!(v > a)) return 0.0f;
-    // v > a: the quotient is positive, so the shader's 0 + (...) * 1 leaves it unchanged
-    return clampf(__fdiv_rn(v - a, 1.0f - a), 0.0f, 1.0f);
+    // v > a: the quotient is positive, so the shader's 0 + (...) * 1 leaves it unchanged. v is at
+    // most 1, so 1 - a is at least 2^-24 and the unscaled division applies.
+    return clampf(div_rn_normal(v - a, 1.0f - a), 0.0f, 1.0f);
 }
 
 // ------------------------------------------------------------------ sampler
@@ -479,7 +481,10 @@ __device__ __forceinline__ float low_erosion(const LowG<FSET>& l, const TexView&
     if constexpr (kSet<FSET> == mm::FSET_PREC) {
         float g = filt3(l.g, Fp8<1>()) * tv.scale[1], b = filt3(l.g, Fp8<2>()) * tv.scale[2],
               a = filt3(l.g, Fp8<3>()) * tv.scale[3];
-        return ((0.625f * g) + (0.25f * b)) + (0.125f * a);
+        const float e = ((0.625f * g) + (0.25f * b)) + (0.125f * a);
+        // the caller's scales may take it past 1, where its remap is 1 whatever the value: cut here, so the
+        // remap's division never sees an infinity
+        return e > 1.0f ? 1.0f : e;
     } else {
         float g, b4, a8;  // power-of-two weights folded into the scale, as in read_hi_erosion
         if (l.g.q8) {
