@@ -144,28 +144,36 @@ __device__ __forceinline__ float remapClamped01(float v, float a) {
 // ------------------------------------------------------------------ sampler
 // x = u * n - 0.5, optionally rounded to 1/256 (fixed-point sub-texel weights), i0 = floor(x) mod n
 // (n a power of two: two's-complement AND is the floor modulo), f = x - floor(x).
-// u * n is exact (n a power of two), so fma(u, n, -0.5) rounds like u * n - 0.5. With the 1/256 rounding,
-// k = floor(x * 256 + 0.5) (x * 256 exact) gives floor(k / 256) = k >> 8 and the fraction
-// (k & 255) / 256 exactly as the float steps do, for texel coordinates below 2^23 in magnitude
-// (8.4 M texels; the presets stay below 1e5). With the rounding, w = (256 - fk) | fk << 16 holds the
-// integer weights of the two texels (fk = k & 255) for the integer filter below. k comes from one
-// v_cvt_flr_i32_f32 (floor and conversion), i0 from one v_bfe_u32 (bits 8 .. 8 + log2 n of k, the
-// same as (k >> 8) & (n - 1) in two's complement); lg = log2 n.
-__device__ __forceinline__ void axis_p2(float u, int n, int lg, int q8, int& i0, float& f, uint32_t& w) {
-    const float x = __builtin_fmaf(u, (float)n, -0.5f);
+// u * n is exact (n a power of two), so fma(u, n, -0.5) rounds like u * n - 0.5, and fma(u, 256 n, -128) is
+// 256 times that with the same rounding. k = floor(256 x + 0.5) gives floor(k / 256) = k >> 8 and the
+// fraction (k & 255) / 256 exactly as the float steps do, for texel coordinates below 2^23 in magnitude
+// (8.4 M texels; the presets stay below 1e5). k comes from one v_cvt_flr_i32_f32 (floor and conversion);
+// 256 n and the literals keep the two float steps full-rate (a scalar 256.0 operand would halve their rate).
+// With the rounding, w = (256 - fk) | fk << 16 holds the integer weights of the two texels (fk = k & 255) for
+// the integer filter below. Returns k (without the rounding, floor(x) * 256): the texel index sits in bits
+// 8 .. 8 + log2 n.
+__device__ __forceinline__ uint32_t axis_p2(float u, int n, int q8, float& f, uint32_t& w) {
+    const float x256 = __builtin_fmaf(u, (float)(n << 8), -128.0f);
     if (q8) {
         int k;
-        asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(k) : "v"(__builtin_fmaf(x, 256.0f, 0.5f)));
-        i0 = (int)__builtin_amdgcn_ubfe((uint32_t)k, 8u, (uint32_t)lg);
+        asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(k) : "v"(x256 + 0.5f));
         const uint32_t fk = (uint32_t)k & 255u;
         f = (float)fk * (1.0f / 256.0f);
         w = __umul24(fk, 65535u) + 256u;  // (256 - fk) | fk << 16
-    } else {
-        const float fl = floorf(x);
-        f = x - fl;
-        i0 = ((int)fl) & (n - 1);
-        w = 0u;
+        return (uint32_t)k;
     }
+    const float x = x256 * (1.0f / 256.0f);
+    const float fl = floorf(x);
+    f = x - fl;
+    w = 0u;
+    return (uint32_t)(int)fl << 8;
+}
+// Texel index of k (one v_bfe_u32; lg = log2 n), and its byte offset along x (a shift and a mask).
+__device__ __forceinline__ uint32_t texel_index(uint32_t k, int lg) { return __builtin_amdgcn_ubfe(k, 8u, (uint32_t)lg); }
+template <int BYTES>
+__device__ __forceinline__ uint32_t texel_offset(uint32_t k, int n) {
+    constexpr int lb = BYTES == 2 ? 1 : BYTES == 4 ? 2 : 3;
+    return (k >> (8 - lb)) & ((uint32_t)(n - 1) << lb);
 }
 
 __device__ __forceinline__ uint32_t ld_u32(const uint8_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
@@ -224,29 +232,29 @@ template <int BYTES> struct G3 {
 };
 
 // Gather of the 2x2 bilinear footprint. APRON: the texture stores n+1 texels per axis with texel n
-// equal to texel 0, so the +1 neighbour never wraps.
+// equal to texel 0, so the +1 neighbour never wraps: every row pair of the footprint is at the same 32-bit
+// byte offset from a uniform base of its own (data, data + one row, + one slice, + both), so one offset -- a
+// shift, a mask and a 24-bit multiply-add per further axis -- serves all its loads, in the scalar-base +
+// vector-offset form with no 64-bit address arithmetic. (Textures are below 4 GiB, checked at the boundary;
+// row and slice strides in bytes fit 24-bit operands: dims <= 8192, slices <= 1025^2 texels of 8 bytes.)
+// An offset per row pair, each with its own multiplies and shift, took 53 issue cycles for a volume, this 24.
 template <int BYTES, bool APRON>
 __device__ __forceinline__ G2<BYTES> gather2(const TexView& tv, float u, float v, int q8) {
     G2<BYTES> g;
     g.q8 = q8;
-    int x0, y0;
-    axis_p2(u, tv.w, tv.lw, q8, x0, g.fx, g.wx);
-    axis_p2(v, tv.h, tv.lh, q8, y0, g.fy, g.wy);
-    int x1, y1;
-    if (APRON) { x1 = x0 + 1; y1 = y0 + 1; }
-    else { x1 = (x0 + 1) & (tv.w - 1); y1 = (y0 + 1) & (tv.h - 1); }
-    // 32-bit byte offsets from the uniform base (textures are below 4 GiB, checked at the boundary):
-    // the loads take the scalar-base + vector-offset form, with no 64-bit address arithmetic
-    // (row and slice products fit 24-bit operands: dims <= 8192, slices <= 1025^2 texels)
-    const uint32_t r0 = __umul24((uint32_t)y0, (uint32_t)tv.stride), r1 = __umul24((uint32_t)y1, (uint32_t)tv.stride);
+    const uint32_t kx = axis_p2(u, tv.w, q8, g.fx, g.wx), ky = axis_p2(v, tv.h, q8, g.fy, g.wy);
+    const uint32_t row = (uint32_t)tv.stride * BYTES;
+    const uint32_t r0 = __umul24(texel_index(ky, tv.lh), row), x0 = texel_offset<BYTES>(kx, tv.w);
     if constexpr (APRON) {
-        ld_pair<BYTES>(tv.data + (r0 + (uint32_t)x0) * BYTES, g.t[0], g.t[1]);
-        ld_pair<BYTES>(tv.data + (r1 + (uint32_t)x0) * BYTES, g.t[2], g.t[3]);
+        const uint32_t o = r0 + x0;
+        ld_pair<BYTES>(tv.data + o, g.t[0], g.t[1]);
+        ld_pair<BYTES>(tv.data + row + o, g.t[2], g.t[3]);
     } else {
-        g.t[0] = ld_texel<BYTES>(tv.data + (r0 + (uint32_t)x0) * BYTES);
-        g.t[1] = ld_texel<BYTES>(tv.data + (r0 + (uint32_t)x1) * BYTES);
-        g.t[2] = ld_texel<BYTES>(tv.data + (r1 + (uint32_t)x0) * BYTES);
-        g.t[3] = ld_texel<BYTES>(tv.data + (r1 + (uint32_t)x1) * BYTES);
+        const uint32_t r1 = __umul24(texel_index(ky + 256u, tv.lh), row), x1 = texel_offset<BYTES>(kx + 256u, tv.w);
+        g.t[0] = ld_texel<BYTES>(tv.data + (r0 + x0));
+        g.t[1] = ld_texel<BYTES>(tv.data + (r0 + x1));
+        g.t[2] = ld_texel<BYTES>(tv.data + (r1 + x0));
+        g.t[3] = ld_texel<BYTES>(tv.data + (r1 + x1));
     }
     return g;
 }
@@ -255,34 +263,31 @@ template <int BYTES, bool APRON>
 __device__ __forceinline__ G3<BYTES> gather3(const TexView& tv, float u, float v, float w, int q8) {
     G3<BYTES> g;
     g.q8 = q8;
-    int x0, y0, z0;
     const int n = tv.w;
-    axis_p2(u, n, tv.lw, q8, x0, g.fx, g.wx);
-    axis_p2(v, n, tv.lw, q8, y0, g.fy, g.wy);
-    axis_p2(w, n, tv.lw, q8, z0, g.fz, g.wz);
-
-    int x1, y1, z1;
-    if (APRON) { x1 = x0 + 1; y1 = y0 + 1; z1 = z0 + 1; }
-    else { x1 = (x0 + 1) & (n - 1); y1 = (y0 + 1) & (n - 1); z1 = (z0 + 1) & (n - 1); }
+    const uint32_t kx = axis_p2(u, n, q8, g.fx, g.wx), ky = axis_p2(v, n, q8, g.fy, g.wy),
+                   kz = axis_p2(w, n, q8, g.fz, g.wz);
+    const uint32_t row = (uint32_t)tv.stride * BYTES, slice = (uint32_t)tv.sliceStride * BYTES;
     const uint8_t* b = tv.data;
-    const uint32_t s0 = __umul24((uint32_t)z0, (uint32_t)tv.sliceStride), s1 = __umul24((uint32_t)z1, (uint32_t)tv.sliceStride);
-    const uint32_t q0 = __umul24((uint32_t)y0, (uint32_t)tv.stride), q1 = __umul24((uint32_t)y1, (uint32_t)tv.stride);
-    const uint32_t r00 = s0 + q0, r10 = s0 + q1, r01 = s1 + q0, r11 = s1 + q1;
-    const uint32_t ux0 = (uint32_t)x0, ux1 = (uint32_t)x1;
+    const uint32_t s0 = __umul24(texel_index(kz, tv.lw), slice), q0 = __umul24(texel_index(ky, tv.lw), row),
+                   x0 = texel_offset<BYTES>(kx, n);
     if constexpr (APRON) {
-        ld_pair<BYTES>(b + (r00 + ux0) * BYTES, g.t[0], g.t[1]);
-        ld_pair<BYTES>(b + (r10 + ux0) * BYTES, g.t[2], g.t[3]);
-        ld_pair<BYTES>(b + (r01 + ux0) * BYTES, g.t[4], g.t[5]);
-        ld_pair<BYTES>(b + (r11 + ux0) * BYTES, g.t[6], g.t[7]);
+        const uint32_t o = s0 + (q0 + x0);
+        ld_pair<BYTES>(b + o, g.t[0], g.t[1]);
+        ld_pair<BYTES>(b + row + o, g.t[2], g.t[3]);
+        ld_pair<BYTES>(b + slice + o, g.t[4], g.t[5]);
+        ld_pair<BYTES>(b + (size_t)(slice + row) + o, g.t[6], g.t[7]);
     } else {
-        g.t[0] = ld_texel<BYTES>(b + (r00 + ux0) * BYTES);
-        g.t[1] = ld_texel<BYTES>(b + (r00 + ux1) * BYTES);
-        g.t[2] = ld_texel<BYTES>(b + (r10 + ux0) * BYTES);
-        g.t[3] = ld_texel<BYTES>(b + (r10 + ux1) * BYTES);
-        g.t[4] = ld_texel<BYTES>(b + (r01 + ux0) * BYTES);
-        g.t[5] = ld_texel<BYTES>(b + (r01 + ux1) * BYTES);
-        g.t[6] = ld_texel<BYTES>(b + (r11 + ux0) * BYTES);
-        g.t[7] = ld_texel<BYTES>(b + (r11 + ux1) * BYTES);
+        const uint32_t s1 = __umul24(texel_index(kz + 256u, tv.lw), slice),
+                       q1 = __umul24(texel_index(ky + 256u, tv.lw), row), x1 = texel_offset<BYTES>(kx + 256u, n);
+        const uint32_t r00 = s0 + q0, r10 = s0 + q1, r01 = s1 + q0, r11 = s1 + q1;
+        g.t[0] = ld_texel<BYTES>(b + (r00 + x0));
+        g.t[1] = ld_texel<BYTES>(b + (r00 + x1));
+        g.t[2] = ld_texel<BYTES>(b + (r10 + x0));
+        g.t[3] = ld_texel<BYTES>(b + (r10 + x1));
+        g.t[4] = ld_texel<BYTES>(b + (r01 + x0));
+        g.t[5] = ld_texel<BYTES>(b + (r01 + x1));
+        g.t[6] = ld_texel<BYTES>(b + (r11 + x0));
+        g.t[7] = ld_texel<BYTES>(b + (r11 + x1));
     }
     return g;
 }
@@ -502,32 +507,69 @@ __device__ __forceinline__ float low_erosion(const LowG<FSET>& l, const TexView&
 }
 
 // ------------------------------------------------------------------ shader functions
+// The launch's constants that every sample uses. A vector instruction with a scalar-register operand issues
+// at half rate (4.3 against 2.5 cycles for an add, multiply or FMA), so those used three times or more by a
+// density sample are kept in vector registers for the whole march: pin() makes the copy opaque, or the
+// compiler would read the scalar register again at each use. With these six the kernels fit in the 80
+// registers of 6 waves per SIMD. Pinning the wind's, the hi-res and curl scales too takes 82 (5 waves):
+// 1080p march + noise 1.560 against 1.540 ms, 16 views 5.14 against 5.02 ms; all of them 1.565 and 5.17. The
+// surrogate's kernels pin none: at their cap of 96 registers each one is a spill around the network's tiles.
+struct HotConsts {
+    float camPos[3], centerY, projRadius, invThickness, windStrength, wind[3], time;
+    float weatherScale, lowScale, curlScale, hiScale;
+    __device__ __forceinline__ V3 cam() const { return ld3(camPos); }
+    __device__ __forceinline__ V3 center() const { return mk(camPos[0], centerY, camPos[2]); }
+};
+template <bool PIN>
+__device__ __forceinline__ float pin(float x) {
+    if (PIN) asm("" : "+v"(x));  // empty: the compiler makes the copy, with the wait states it needs
+    return x;
+}
+template <bool PIN>
+__device__ __forceinline__ HotConsts hot_consts(const MarchConsts& c) {
+    HotConsts h;
+    h.camPos[0] = pin<PIN>(c.camPos[0]); h.camPos[1] = c.camPos[1]; h.camPos[2] = pin<PIN>(c.camPos[2]);
+    h.centerY = pin<PIN>(c.earthCenter[1]);
+    h.projRadius = pin<PIN>(c.projRadius);
+    h.invThickness = c.invThickness;
+    h.windStrength = c.windStrength;
+    h.wind[0] = c.wind[0]; h.wind[1] = c.wind[1]; h.wind[2] = c.wind[2];
+    h.time = c.time;
+    h.weatherScale = pin<PIN>(c.weatherScale); h.lowScale = pin<PIN>(c.lowScale);
+    h.curlScale = c.curlScale; h.hiScale = c.hiScale;
+    return h;
+}
+
 // getProjectedShellPoint (comp:180-182)
-__device__ __forceinline__ V3 proj_shell(const MarchConsts& c, V3 pt, V3 center) {
+__device__ __forceinline__ V3 proj_shell(const HotConsts& c, V3 pt, V3 center) {
     return (c.projRadius * normalize3(pt - center)) + center;
 }
 // getRelativeHeight (comp:186-188)
-__device__ __forceinline__ float rel_height(const MarchConsts& c, V3 pt, V3 proj) {
+__device__ __forceinline__ float rel_height(const HotConsts& c, V3 pt, V3 proj) {
     return clampf(length3(pt - proj) * c.invThickness, 0.0f, 1.0f);
 }
 
-// cloudLayerDensity (comp:193-204)
-__device__ __forceinline__ float layer_density(float h, float type) {
-    h = clampf(h, 0.0f, 1.0f);
+// cloudLayerDensity (comp:193-204) over 8, for a relative height already clamped to [0, 1]. The profiles
+// peak at 5.1, so an eighth of each lies in [0, 1] and its max(0, .) is the clamp modifier of the product
+// (free; a v_max costs 4.3 cycles, and there are three). Scaling by a power of two commutes with every
+// rounding here: the caller's density is 8 times this times the shape, exactly.
+constexpr float kLayerScale = 8.0f;
+__device__ __forceinline__ float layer_density8(float h, float type) {
     // remap(h, 0, b, 0, 1) = 0 + h (1 / b): the 0 + only turns a -0 into +0, and these factors meet
     // only products, max(0, .) and mixes whose zero signs never reach a nonzero profile (the caller
     // tests the profile against 0)
-    const float r02 = h * (1.0f / 0.2f);
-    float cumulus = fmaxf(0.0f, r02 * remapk(h, 0.7f, 1.0f / (0.9f - 0.7f), 1.0f, -1.0f));
-    float strato = fmaxf(0.0f, r02 * remapk(h, 0.2f, 1.0f / (0.7f - 0.2f), 1.0f, -1.0f));
-    float stratus = fmaxf(0.0f, (h * (1.0f / 0.1f)) * remapk(h, 0.2f, 1.0f / (0.3f - 0.2f), 1.0f, -1.0f));
+    const float r02 = h * ((1.0f / 0.2f) / kLayerScale);
+    float cumulus = clampf(r02 * remapk(h, 0.7f, 1.0f / (0.9f - 0.7f), 1.0f, -1.0f), 0.0f, 1.0f);
+    float strato = clampf(r02 * remapk(h, 0.2f, 1.0f / (0.7f - 0.2f), 1.0f, -1.0f), 0.0f, 1.0f);
+    float stratus = clampf((h * ((1.0f / 0.1f) / kLayerScale)) * remapk(h, 0.2f, 1.0f / (0.3f - 0.2f), 1.0f, -1.0f),
+                           0.0f, 1.0f);
     float d1 = mixf(stratus, strato, clampf(type * 2.0f, 0.0f, 1.0f));
     float d2 = mixf(strato, cumulus, clampf((type - 0.5f) * 2.0f, 0.0f, 1.0f));
     return mixf(d1, d2, type);
 }
 
 // wind offset (comp:414, 445)
-__device__ __forceinline__ V3 wind_offset(const MarchConsts& c, float h) {
+__device__ __forceinline__ V3 wind_offset(const HotConsts& c, float h) {
     // h is a clamped relative height in [0, 1], so h * 0 is a zero
     V3 w = mk(c.wind[0] + h * 0.1f, c.wind[1] + h * 0.05f, c.wind[2] + 0.0f);
     return (c.windStrength * w) * (c.time + h * 200.0f);
@@ -536,11 +578,11 @@ __device__ __forceinline__ V3 wind_offset(const MarchConsts& c, float h) {
 // The light-cone surrogate's density probes only feed the network (the recorder of its training
 // rows takes the same probes), so they use the hardware square root, reciprocal square root,
 // reciprocal, exp2 and log2 (about 1 ulp) without the rounding fix-ups of the march's own samples.
-__device__ __forceinline__ V3 proj_shell_fast(const MarchConsts& c, V3 pt, V3 center) {
+__device__ __forceinline__ V3 proj_shell_fast(const HotConsts& c, V3 pt, V3 center) {
     const V3 d = pt - center;
     return (c.projRadius * (d * __builtin_amdgcn_rsqf(dot3(d, d)))) + center;
 }
-__device__ __forceinline__ float rel_height_fast(const MarchConsts& c, V3 pt, V3 proj) {
+__device__ __forceinline__ float rel_height_fast(const HotConsts& c, V3 pt, V3 proj) {
     const V3 d = pt - proj;
     return clampf(__builtin_amdgcn_sqrtf(dot3(d, d)) * c.invThickness, 0.0f, 1.0f);
 }
@@ -551,35 +593,37 @@ __device__ __forceinline__ float remapClamped01_fast(float v, float a) {
 // wout (optional) receives the weather coverage and type the test read (left untouched when the
 // height skips the read). EXACT = false: the surrogate probes' arithmetic (proj_shell_fast above).
 template <int FSET, bool COUNT, bool EXACT = true>
-__device__ __forceinline__ float cloud_test(const MarchConsts& c, const MarchTextures& tx, V3 pos, float h, V3 center,
+__device__ __forceinline__ float cloud_test(const HotConsts& c, const MarchTextures& tx, V3 pos, float h, V3 center,
                                             Tally& nd, Weather* wout = nullptr) {
     if (COUNT) nd++;
     // every layer profile is 0 at h = 0 and below 1e-7 for h >= 0.9 (the cumulus top; stratocumulus
     // and stratus end at 0.7 and 0.3), for any cloud type in [0, 1]: the density test below would
     // return 0 there whatever the textures hold, so the weather and low-res reads are skipped
-    if (!(h > 0.0f && h < 0.9f)) return 0.0f;
+    // (h is clamped, never negative: one unsigned compare of its bits tests both ends)
+    if (__float_as_uint(h) - 1u >= __float_as_uint(0.9f) - 1u) return 0.0f;
     if (COUNT) nd += kTallyWeather;
     constexpr int q8 = kQ8<FSET>;
     V3 proj = EXACT ? proj_shell(c, pos, center) : proj_shell_fast(c, pos, center);
     Weather w = read_weather<FSET>(tx.weather, c.weatherScale * (proj.x - c.camPos[0]),
                                    c.weatherScale * (proj.z - c.camPos[2]), q8);
     if (wout) *wout = w;
-    float layer = layer_density(h, w.type);
+    const float layer8 = layer_density8(h, w.type);
     // density = layer * remapClamped(R, ...) with the remap in [0, 1]: a zero layer density gives 0
     // whatever the low-res texel, so its gather is skipped (comp:240-243 evaluate to the same 0)
-    if (layer == 0.0f) return 0.0f;
+    if (layer8 == 0.0f) return 0.0f;
     if (COUNT) nd += kTallyLow;
     LowG<FSET> lg = gather_low<FSET>(tx.low, pos * c.lowScale, q8);
     float shape = low_shape<FSET>(lg, tx.low);
     // remapClamped(shape, 0.3, 1, 0, 1); its 0 + (.) only flips the sign of a zero, which the
     // < 0.0001 test below treats alike
-    float density = layer * clampf((shape - 0.3f) * (1.0f / (1.0f - 0.3f)), 0.0f, 1.0f);
-    if (density < 0.0001f) return 0.0f;
+    const float density8 = layer8 * clampf((shape - 0.3f) * (1.0f / (1.0f - 0.3f)), 0.0f, 1.0f);
+    if (density8 < 0.0001f / kLayerScale) return 0.0f;
     // remapClamped(density, erosion, 1, 0, 1) with erosion in [0, 1] is exactly 1 for density > 1:
     // (density - erosion) and (1 - erosion) round monotonically, so their quotient is >= 1 (or +inf
     // for erosion = 1) and the clamp returns 1. The layer profile reaches 5, so dense cloud interiors
     // skip the erosion channels, the coverage pow and both remap quotients.
-    if (density > 1.0f) return 1.0f;
+    if (density8 > 1.0f / kLayerScale) return 1.0f;
+    const float density = density8 * kLayerScale;
     // heightBiasCoverage(relativeHeight, min(0.85, cloudInfo.r)) (comp:206-208, 245)
     float e = clampf(remapk(fminf(0.85f, w.coverage), 0.7f, 1.0f / (0.8f - 0.7f), 1.0f, 0.8f - 1.0f), 0.8f, 1.0f);
     float erosion = low_erosion<FSET>(lg, tx.low);
@@ -590,7 +634,7 @@ __device__ __forceinline__ float cloud_test(const MarchConsts& c, const MarchTex
 }
 
 template <int FSET, bool COUNT>
-__device__ __forceinline__ float cloud_hires(const MarchConsts& c, const MarchTextures& tx, V3 pos, float curlStrength,
+__device__ __forceinline__ float cloud_hires(const HotConsts& c, const MarchTextures& tx, V3 pos, float curlStrength,
                                              float orig, float h, int& nh) {
     if (COUNT) nh++;
     constexpr int q8 = kQ8<FSET>;
@@ -764,7 +808,7 @@ __device__ __forceinline__ RaySetup ray_setup(const MarchConsts& c, const MarchT
         V3 rrd = ((c0 * rd.x) + (c1 * rd.y)) + (c2 * rd.z);
         V3 rro = ((c0 * camPos.x) + (c1 * camPos.y)) + (c2 * camPos.z);
         V3 point = (rrd * r.tEnd) + rro;
-        V3 pr = proj_shell(c, point, center);
+        V3 pr = proj_shell(hot_consts<false>(c), point, center);
         float u = 0.00002f * (pr.x - camPos.x) + 0.35f;
         float v = 0.00002f * (pr.z - camPos.z) + 0.35f;
         V3 bg = night_sky(c, tx, u, v);
@@ -813,20 +857,19 @@ __device__ __forceinline__ float4 compose(const MarchConsts& c, const RaySetup& 
 
 // Density along the sun: the six-sample light cone (comp:440-453).
 template <int FSET, bool COUNT>
-__device__ __forceinline__ float cone_dal(const MarchConsts& c, const MarchTextures& tx, V3 currentPos, float stepSize,
+__device__ __forceinline__ float cone_dal(const MarchConsts& c, const HotConsts& h, const MarchTextures& tx, V3 currentPos, float stepSize,
                                           Tally& nd, int& nh) {
-    V3 center = ld3(c.camPos);
-    center.y = c.earthCenter[1];
+    const V3 center = h.center();
     float dal = 0.0f;
     // two independent samples in flight per lane (unrolling all six is slower: code size)
 #pragma unroll 2
     for (int i = 0; i < 6; i++) {
         V3 lsPos = currentPos + ((3.0f * stepSize) * ld3(c.coneOffsets[i]));
-        V3 lsProj = proj_shell(c, lsPos, center);
-        float lsHeight = rel_height(c, lsPos, lsProj);
-        V3 lwo = wind_offset(c, lsHeight);
-        float ls = cloud_test<FSET, COUNT>(c, tx, lsPos + lwo, lsHeight, center, nd);
-        if (ls > 0.0f) dal += cloud_hires<FSET, COUNT>(c, tx, lsPos + lwo, stepSize, ls, lsHeight, nh);
+        V3 lsProj = proj_shell(h, lsPos, center);
+        float lsHeight = rel_height(h, lsPos, lsProj);
+        V3 lwo = wind_offset(h, lsHeight);
+        float ls = cloud_test<FSET, COUNT>(h, tx, lsPos + lwo, lsHeight, center, nd);
+        if (ls > 0.0f) dal += cloud_hires<FSET, COUNT>(h, tx, lsPos + lwo, stepSize, ls, lsHeight, nh);
     }
     return dal;
 }
@@ -847,19 +890,18 @@ __device__ __forceinline__ float beers_of(float dal, float beerBlend) {
 // The coverage and type are those the hit's own density test read (the weather map at the
 // projection of the wind-offset hit position), carried in the job queue.
 template <int FSET, bool COUNT>
-__device__ __forceinline__ void cone_features(const MarchConsts& c, const MarchTextures& tx, V3 pos, float stepSize,
+__device__ __forceinline__ void cone_features(const MarchConsts& c, const HotConsts& h, const MarchTextures& tx, V3 pos, float stepSize,
                                               float rh, float lo, float dens, float cov, float type, float* f,
                                               Tally& nd) {
-    V3 center = ld3(c.camPos);
-    center.y = c.earthCenter[1];
-    const V3 p = pos + wind_offset(c, rh);
+    const V3 center = h.center();
+    const V3 p = pos + wind_offset(h, rh);
     f[0] = rh; f[1] = lo; f[2] = dens; f[3] = cov; f[4] = type; f[5] = c.sunDir[1];
 #pragma unroll 1
     for (int i = 0; i < 3; i++) {
         V3 lsPos = pos + ((3.0f * stepSize) * ld3(c.probeOffsets[i]));
-        V3 lsProj = proj_shell_fast(c, lsPos, center);
-        float lsHeight = rel_height_fast(c, lsPos, lsProj);
-        f[6 + i] = cloud_test<FSET, COUNT, false>(c, tx, lsPos + wind_offset(c, lsHeight), lsHeight, center, nd);
+        V3 lsProj = proj_shell_fast(h, lsPos, center);
+        float lsHeight = rel_height_fast(h, lsPos, lsProj);
+        f[6 + i] = cloud_test<FSET, COUNT, false>(h, tx, lsPos + wind_offset(h, lsHeight), lsHeight, center, nd);
     }
     f[9] = stepSize * c.invThickness;
     const float k = 6.283185307179586f * c.hiScale;
@@ -905,21 +947,19 @@ struct TripSample {
 };
 
 template <int FSET, bool COUNT, bool KEEPW = false>
-__device__ __forceinline__ TripSample trip_eval(const MarchConsts& c, const MarchTextures& tx, const RaySetup& r,
+__device__ __forceinline__ TripSample trip_eval(const MarchConsts& c, const HotConsts& h, const MarchTextures& tx, const RaySetup& r,
                                                 bool noHits, float stepSize, float t) {
     TripSample s;
     s.nd = s.nh = 0;
     s.w.coverage = s.w.type = 0.0f;
-    const V3 camPos = ld3(c.camPos);
-    V3 center = camPos;
-    center.y = c.earthCenter[1];
-    s.pos = camPos + (t * r.rd);
-    const V3 proj = proj_shell(c, s.pos, center);
-    s.rHeight = rel_height(c, s.pos, proj);
-    const V3 wo = wind_offset(c, s.rHeight);
-    s.lo = cloud_test<FSET, COUNT>(c, tx, s.pos + wo, s.rHeight, center, s.nd, KEEPW ? &s.w : nullptr);
+    const V3 center = h.center();
+    s.pos = h.cam() + (t * r.rd);
+    const V3 proj = proj_shell(h, s.pos, center);
+    s.rHeight = rel_height(h, s.pos, proj);
+    const V3 wo = wind_offset(h, s.rHeight);
+    s.lo = cloud_test<FSET, COUNT>(h, tx, s.pos + wo, s.rHeight, center, s.nd, KEEPW ? &s.w : nullptr);
     s.dens = s.lo;
-    if (s.lo > 0.0f && !noHits) s.dens = cloud_hires<FSET, COUNT>(c, tx, s.pos + wo, stepSize, s.lo, s.rHeight, s.nh);
+    if (s.lo > 0.0f && !noHits) s.dens = cloud_hires<FSET, COUNT>(h, tx, s.pos + wo, stepSize, s.lo, s.rHeight, s.nh);
     return s;
 }
 
@@ -990,12 +1030,12 @@ __device__ __forceinline__ bool trip_commit(const MarchConsts& c, const RaySetup
 
 // One trip of the reference's for-loop: its samples, then its state update.
 template <int FSET, bool COUNT, bool KEEPW = false>
-__device__ __forceinline__ bool march_trip(const MarchConsts& c, const MarchTextures& tx, const RaySetup& r,
+__device__ __forceinline__ bool march_trip(const MarchConsts& c, const HotConsts& h, const MarchTextures& tx, const RaySetup& r,
                                            MarchState& m, V3& jobPos, float& jobStep, float& jobX0, float& jobW,
                                            float& jobRh, float& jobLo, float& jobDens, Weather& jobWeather, Tally& nd,
                                            int& nh) {
     if (!trip_begin<FSET>(c, m)) return false;
-    const TripSample s = trip_eval<FSET, COUNT, KEEPW>(c, tx, r, m.noHits, m.stepSize, m.t);
+    const TripSample s = trip_eval<FSET, COUNT, KEEPW>(c, h, tx, r, m.noHits, m.stepSize, m.t);
     const float step = m.stepSize;
     const bool job = trip_commit<FSET>(c, r, m, s.lo, s.dens, jobW);
     if (job) {
@@ -1099,6 +1139,7 @@ __global__ __launch_bounds__(64) void march_kernel(const MarchConsts c, const Ma
     if (gi >= c.gridW || gj >= c.gridH) return;
     int px, py;
     tile_pixel(c, gi, gj, px, py);
+    const HotConsts h = hot_consts<true>(c);
     Tally nd = 0;
     int nh = 0, nj = 0, nc = 0;  // density, detail samples; cone jobs, jobs on the plain cone
     const RaySetup r = ray_setup(c, tx, px, py);
@@ -1116,8 +1157,8 @@ __global__ __launch_bounds__(64) void march_kernel(const MarchConsts c, const Ma
         V3 jp;
         float js, jx0, jw, jrh, jlo, jd;
         Weather jwe;
-        if (march_trip<FSET, COUNT>(c, tx, r, m, jp, js, jx0, jw, jrh, jlo, jd, jwe, nd, nh)) {
-            float dal = cone_dal<FSET, COUNT>(c, tx, jp, js, nd, nh);
+        if (march_trip<FSET, COUNT>(c, h, tx, r, m, jp, js, jx0, jw, jrh, jlo, jd, jwe, nd, nh)) {
+            float dal = cone_dal<FSET, COUNT>(c, h, tx, jp, js, nd, nh);
             transmittance = mixf(transmittance, jx0 * beers_of(dal, r.beerBlend), jw);
             if (COUNT) { nj++; nc++; }
         }
@@ -1169,7 +1210,7 @@ __device__ __forceinline__ uint32_t mix32(uint32_t x) {
 // myBlend is the calling lane's own Beer blend; a job's blend is its owner's, fetched by a lane
 // shuffle rather than stored in the queue.
 template <int FSET, bool COUNT, int MODE, class Q>
-__device__ __forceinline__ void run_batch(const MarchConsts& c, const MarchTextures& tx, Q& q, const int nb,
+__device__ __forceinline__ void run_batch(const MarchConsts& c, const HotConsts& h, const MarchTextures& tx, Q& q, const int nb,
                                           const float myBlend, Tally& nd, int& nh, int& nj, int& nc) {
     const int lane = threadIdx.x;
     const float blend = __shfl(myBlend, q.owner[lane]);  // every lane takes part; slots >= nb are unused
@@ -1177,7 +1218,7 @@ __device__ __forceinline__ void run_batch(const MarchConsts& c, const MarchTextu
     if constexpr (MODE == CONE_PLAIN) {
         if (COUNT) nc += nb;
         if (lane < nb) {
-            float dal = cone_dal<FSET, COUNT>(c, tx, mk(q.x[lane], q.y[lane], q.z[lane]), q.step[lane], nd, nh);
+            float dal = cone_dal<FSET, COUNT>(c, h, tx, mk(q.x[lane], q.y[lane], q.z[lane]), q.step[lane], nd, nh);
             q.res[lane] = q.x0[lane] * beers_of(dal, blend);
         }
     } else if constexpr (MODE == CONE_COLLECT) {
@@ -1188,13 +1229,13 @@ __device__ __forceinline__ void run_batch(const MarchConsts& c, const MarchTextu
         bool keep = false;
         if (lane < nb) {
             const V3 pos = mk(q.x[lane], q.y[lane], q.z[lane]);
-            dal = cone_dal<FSET, COUNT>(c, tx, pos, q.step[lane], nd, nh);
+            dal = cone_dal<FSET, COUNT>(c, h, tx, pos, q.step[lane], nd, nh);
             q.res[lane] = q.x0[lane] * beers_of(dal, blend);
             const uint32_t hsh = mix32(__float_as_uint(pos.x) ^ mix32(__float_as_uint(pos.y) ^
                                        mix32(__float_as_uint(pos.z) ^ c.collectSeed)));
             keep = (hsh % c.collectKeep) == 0u;
             if (keep)
-                cone_features<FSET, COUNT>(c, tx, pos, q.step[lane], q.rh[lane], q.lo[lane], q.dens[lane], q.cov[lane],
+                cone_features<FSET, COUNT>(c, h, tx, pos, q.step[lane], q.rh[lane], q.lo[lane], q.dens[lane], q.cov[lane],
                                            q.type[lane], f, nd);
         }
         const unsigned long long km = __ballot(keep);
@@ -1217,7 +1258,7 @@ __device__ __forceinline__ void run_batch(const MarchConsts& c, const MarchTextu
         float f[surr::kIn];
         for (int k = 0; k < surr::kIn; k++) f[k] = 0.0f;
         if (lane < nb)
-            cone_features<FSET, COUNT>(c, tx, mk(q.x[lane], q.y[lane], q.z[lane]), q.step[lane], q.rh[lane],
+            cone_features<FSET, COUNT>(c, h, tx, mk(q.x[lane], q.y[lane], q.z[lane]), q.step[lane], q.rh[lane],
                                        q.lo[lane], q.dens[lane], q.cov[lane], q.type[lane], f, nd);
         for (int k = 0; k < surr::kIn; k++) f[k] = (f[k] - c.surrStats[k]) * c.surrStats[16 + k];
         const surr::FwdOut o = surr::mlp_infer64_h(c.surrFrags, c.surrParams + surr::oB4, f, nb);
@@ -1231,7 +1272,7 @@ __device__ __forceinline__ void run_batch(const MarchConsts& c, const MarchTextu
         if (COUNT) nc += nf;
         if (lane < nf) {
             const int j = q.fallback[lane];
-            q.dal[j] = cone_dal<FSET, COUNT>(c, tx, mk(q.x[j], q.y[j], q.z[j]), q.step[j], nd, nh);
+            q.dal[j] = cone_dal<FSET, COUNT>(c, h, tx, mk(q.x[j], q.y[j], q.z[j]), q.step[j], nd, nh);
         }
         __syncthreads();
         if (lane < nb) {
@@ -1274,6 +1315,7 @@ __device__ __forceinline__ void march_tile(const MarchConsts& c, const MarchText
     const bool valid = gi < c.gridW && gj < c.gridH;
     int px = 0, py = 0;
     if (valid) tile_pixel(c, gi, gj, px, py);
+    const HotConsts h = hot_consts<MODE != CONE_SURROGATE>(c);
     Tally nd = 0;
     int nh = 0, nj = 0, nc = 0;  // density, detail samples; cone jobs, jobs on the plain cone
     RaySetup r;
@@ -1297,7 +1339,7 @@ __device__ __forceinline__ void march_tile(const MarchConsts& c, const MarchText
             jwe.coverage = jwe.type = 0.0f;
             bool job = false;
             if (m.active)
-                job = march_trip<FSET, COUNT, MODE != CONE_PLAIN>(c, tx, r, m, jp, js, jx0, jw, jrh, jlo, jd, jwe, nd, nh);
+                job = march_trip<FSET, COUNT, MODE != CONE_PLAIN>(c, h, tx, r, m, jp, js, jx0, jw, jrh, jlo, jd, jwe, nd, nh);
             const unsigned long long mask = __ballot(job);
             if (job) {
                 const int slot = qn + __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
@@ -1315,7 +1357,7 @@ __device__ __forceinline__ void march_tile(const MarchConsts& c, const MarchText
         if (qn == 0) break;
         __syncthreads();
         const int nb = qn < 64 ? qn : 64;
-        run_batch<FSET, COUNT, MODE>(c, tx, q, nb, valid ? r.beerBlend : 0.0f, nd, nh, nj, nc);
+        run_batch<FSET, COUNT, MODE>(c, h, tx, q, nb, valid ? r.beerBlend : 0.0f, nd, nh, nj, nc);
         for (int s = 0; s < nb; s++)
             if (q.owner[s] == lane) transmittance = mixf(transmittance, q.res[s], q.w[s]);
         queue_shift(q, nb, qn - nb);
@@ -1333,8 +1375,14 @@ __device__ __forceinline__ void march_tile(const MarchConsts& c, const MarchText
     }
 }
 
+// Waves per SIMD the plain marches hold their registers to (80 of them): one lane per ray and no counters, the
+// kernels of full frames and view sets. Left alone they take 83 (96 in the PREC set) and run at 5 waves:
+// 1080p march + noise 1.42 against 1.39 ms. One to three registers spill, outside the sample's code.
+constexpr int kPlainWaves = 6;
+
 template <int FSET, bool COUNT, int MODE>
-__global__ __launch_bounds__(64) void march_batched_kernel(const MarchConsts c, const MarchTextures tx,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE == CONE_PLAIN && !COUNT ? kPlainWaves : 1)))
+void march_batched_kernel(const MarchConsts c, const MarchTextures tx,
                                                            float* __restrict__ out,
                                                            unsigned long long* __restrict__ counts) {
     const int tile = block_tile(c);
@@ -1454,6 +1502,7 @@ __device__ __forceinline__ void march_rp_tile(const MarchConsts& c, const MarchT
     const bool valid = gi < c.gridW && gj < c.gridH;
     int px = 0, py = 0;
     if (valid) tile_pixel(c, gi, gj, px, py);
+    const HotConsts h = hot_consts<MODE != CONE_SURROGATE>(c);
     Tally nd = 0;
     int nh = 0, nj = 0, nc = 0;
     RaySetup r;
@@ -1478,7 +1527,7 @@ __device__ __forceinline__ void march_rp_tile(const MarchConsts& c, const MarchT
             s.pos = mk(0.f, 0.f, 0.f);
             s.rHeight = s.lo = s.dens = 0.0f;
             s.nd = s.nh = 0;
-            if (m.active) s = trip_eval<FSET, COUNT, MODE != CONE_PLAIN>(c, tx, r, m.noHits, step0, tk);
+            if (m.active) s = trip_eval<FSET, COUNT, MODE != CONE_PLAIN>(c, h, tx, r, m.noHits, step0, tk);
             bool mine;  // this lane's trip committed with a light-cone job
             float jw;
             const bool took = commit_round<FSET, LPR>(c, r, m, k, first, tk, s.lo, s.dens, mine, jw);
@@ -1500,7 +1549,7 @@ __device__ __forceinline__ void march_rp_tile(const MarchConsts& c, const MarchT
         if (qn == 0) break;
         __syncthreads();
         const int nb = qn < 64 ? qn : 64;
-        run_batch<FSET, COUNT, MODE>(c, tx, q, nb, valid ? r.beerBlend : 0.0f, nd, nh, nj, nc);
+        run_batch<FSET, COUNT, MODE>(c, h, tx, q, nb, valid ? r.beerBlend : 0.0f, nd, nh, nj, nc);
         for (int j = 0; j < nb; j++)
             if (q.owner[j] / LPR == ray) transmittance = mixf(transmittance, q.res[j], q.w[j]);
         queue_shift(q, nb, qn - nb);
@@ -1662,7 +1711,7 @@ __device__ __forceinline__ void views_group(const ViewDesc* __restrict__ views, 
 }
 
 template <int FSET, bool COUNT, int MODE, int LPR>
-__global__ __launch_bounds__(64)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPR == 1 && !COUNT ? kPlainWaves : 1)))
 void march_views_kernel(const ViewDesc* __restrict__ views, int nViews, const MarchTextures tx, int total,
                         unsigned long long* __restrict__ counts, const int* __restrict__ order,
                         unsigned* __restrict__ sched) {
