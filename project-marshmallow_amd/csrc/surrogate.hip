@@ -7,6 +7,7 @@
 // second term with the residual held fixed.
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <algorithm>
 #include "mm_internal.hpp"
 #include "surrogate_dev.hpp"
 
@@ -157,199 +158,316 @@ __global__ void pack_kernel(const float* __restrict__ p, uint4* __restrict__ fra
     frags[t] = __builtin_bit_cast(uint4, b);
 }
 
-// One Adam step's gradients over a batch: block = one wave = 64 random samples (two 32-sample
-// tiles). Forward in registers (pre-activations parked in LDS), backward dA = W dZ with the same
-// fragment layout, weight gradients dW^T = dZ^T a^T from LDS-transposed tiles, accumulated into
-// the global FP32 gradient buffer with atomics.
-struct TrainLds {
-    float z[2][3][2][16][64];          // [tile][layer][m-tile][acc][lane] pre-activations
-    __bf16 dz[64][40];                 // dZ^T rows = units, 32 samples (+pad)
-    __bf16 act[64][40];                // a^T rows = input units/features, 32 samples (+pad)
-    float x[64][kIn];                  // normalised inputs of the 64 samples
-    float dout[64][2];
+// ---------------------------------------------------------------- training
+// Gradients of a batch: a block of four waves takes 128 rows, 32 per wave. Each wave runs its rows' forward
+// and backward passes in registers (pre-activations included: one wave per SIMD may use them all) and leaves
+// the activations and dZ of every layer in LDS, transposed to [unit][row] in BF16. After one barrier the
+// four waves share the weight gradients dW^T = dZ^T a^T, a 32x32 tile of dW2 and of dW3 and two of the smaller
+// tiles each, over all 128 rows, in MFMA accumulators that persist over the blocks of rows a workgroup takes.
+// The bias gradients are products with ones (dW1's 17th column; tiles of their own for layers 2 and 3).
+//
+// A step is bound by latency, not by its 15 MFLOP: 64 workgroups at the configured batch, each a chain of about
+// 75 MFMAs per wave. One wave per 64 rows with the gradients added by atomics from every 32-row tile (2.4 M
+// device-scope atomics a step) and separate clearing, Adam and packing launches took 146 us a step; this takes
+// 11.5 us and the update 4. The gradient of 500 000 rows: 6.4 ms before, 0.19 ms. The weights go through LDS once
+// per workgroup: each wave loading its own fragments into registers took 15.7 us (144 of them, the rest in
+// accumulator registers at a move per use).
+constexpr int kTrainRows = 128, kTrainWaves = kTrainRows / 32;
+constexpr int kRowPitch = kTrainRows + 8;  // 16 bytes of padding: the 32 lanes' 16-byte reads spread over the banks
+constexpr int kMaxTrainBlocks = 256;       // one per CU; larger batches loop
+constexpr int kPartial = (kParams + 1 + 15) / 16 * 16;  // a workgroup's gradients and loss, floats
+static_assert(kTrainWaves == 4 && kFrags % kTrainWaves == 0, "the tiles' split");
+
+struct alignas(16) TrainLds {
+    __bf16 act[3][kHidden][kRowPitch];  // activations of layers 1 to 3
+    __bf16 dz[3][kHidden][kRowPitch];
+    __bf16 x[32][kRowPitch];            // inputs; row 16 is ones, the rest unused
+    __bf16 dz4[kOut][kRowPitch];
+    uint4 frag[kFrags * 64];            // the weights, loaded once for the four waves
+    float bias[3][kHidden];
+    float red[kTrainWaves][3];
 };
 
-__global__ __launch_bounds__(64) void train_kernel(const float* __restrict__ samples, int n, int stride,
-                                                   const float* __restrict__ params, const float* __restrict__ stats,
-                                                   const uint4* __restrict__ frags, float* __restrict__ grads,
-                                                   float* __restrict__ loss_acc, uint32_t seed, int step,
-                                                   int sequential, float invB) {
-    __shared__ TrainLds L;
-    const int lane = threadIdx.x, h = lane >> 5, c = lane & 31;
-    // rows: a seeded hash draw (training) or rows blockIdx * 64 + lane < n (exact mean gradient)
-    uint32_t idx;
-    bool valid = true;
-    if (sequential) {
-        idx = blockIdx.x * 64u + lane;
-        valid = idx < (uint32_t)n;
-        if (!valid) idx = 0;
+// Gradient sink: a workgroup's own partial buffer (plain stores) or a shared buffer (atomics).
+template <bool ATOMIC>
+__device__ __forceinline__ void put(float* g, int i, float v) {
+    if (ATOMIC) atomicAdd(&g[i], v);
+    else g[i] = v;
+}
+template <bool ATOMIC>
+__device__ __forceinline__ void put4(float* g, int i, const f32x16& a, int r) {  // i a multiple of 4
+    if (ATOMIC) {
+        for (int k = 0; k < 4; k++) atomicAdd(&g[i + k], a[r + k]);
     } else {
-        idx = hash_u32(seed ^ hash_u32((uint32_t)step * 0x632BE5ABu + blockIdx.x * 64u + lane)) % (uint32_t)n;
+        *reinterpret_cast<float4*>(g + i) = make_float4(a[r], a[r + 1], a[r + 2], a[r + 3]);
     }
-    float x[kIn];
-    for (int k = 0; k < kIn; k++) {
-        x[k] = (samples[(size_t)idx * stride + k] - stats[k]) * stats[16 + k];
-        L.x[lane][k] = x[k];
-    }
-    const float D = samples[(size_t)idx * stride + kIn];
-    const float T = __expf(-D);
-    const float rowW = valid ? 1.0f : 0.0f;
-    __syncthreads();
-
-    float lossv = 0.0f;
-    for (int tile = 0; tile < 2; tile++) {
-        // B operand of layer 1 for this tile: features 8h..8h+7 of sample 32*tile + c
-        float xb[8];
-        for (int j = 0; j < 8; j++) xb[j] = L.x[32 * tile + c][8 * h + j];
-        float zs[96];
-        FwdOut o = mlp_forward_tile(frags, params, pack8(xb), zs);
-        for (int l = 0; l < 3; l++)
-            for (int mt = 0; mt < 2; mt++)
-                for (int r = 0; r < 16; r++) L.z[tile][l][mt][r][lane] = zs[(l * 2 + mt) * 16 + r];
-        // loss gradient for sample 32*tile + c (its outputs are held by lanes of half 0)
-        const float Ts = __shfl(T, 32 * tile + c);  // all lanes shuffle; the target lives in lane s
-        const float ws = __shfl(rowW, 32 * tile + c);
-        if (h == 0) {
-            const int s = 32 * tile + c;
-            const float p = __expf(o.o0), r = p - Ts, ar = fabsf(r);
-            const float e = softplus(o.o1), sig = 1.0f / (1.0f + __expf(-o.o1));
-            lossv += ws * (r * r + (e - ar) * (e - ar));
-            L.dout[s][0] = ws * (2.0f * r * p);
-            L.dout[s][1] = ws * (2.0f * (e - ar) * sig);
-        }
-    }
-    __syncthreads();
-
-    for (int tile = 0; tile < 2; tile++) {
-        // ---- layer 4: dZ4^T (2 rows) as B operand of dA3 = W4 dZ4 (k = outputs 8h + j)
-        float dz4[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (h == 0) {
-            dz4[0] = L.dout[32 * tile + c][0] * invB;
-            dz4[1] = L.dout[32 * tile + c][1] * invB;
-        }
-        // dW4^T[u][k] = sum_s dZ4[u][s] a3[k][s], db4: accumulate directly (2 outputs x 64 units)
-        // a3 = hswish(z3) of this lane's sample c for units crow(r, h) + 32 mt
-        {
-            // write a3^T and dz4^T tiles to LDS
-            for (int mt = 0; mt < 2; mt++)
-                for (int r = 0; r < 16; r++)
-                    L.act[mt * 32 + crow(r, h)][c] = (__bf16)hswish(L.z[tile][2][mt][r][lane]);
-            if (h == 0) {
-                L.dz[0][c] = (__bf16)dz4[0];
-                L.dz[1][c] = (__bf16)dz4[1];
-            }
-            __syncthreads();
-            // dW4: M = 2 outputs (rows of dz, padded to 32 with zero rows), N = 64 units, K = 32 samples
-            for (int nt = 0; nt < 2; nt++) {
-                f32x16 acc = {};
-                for (int kt = 0; kt < 2; kt++) {
-                    float a8[8], b8[8];
-                    for (int j = 0; j < 8; j++) {
-                        a8[j] = c < kOut ? (float)L.dz[c][16 * kt + 8 * h + j] : 0.0f;
-                        b8[j] = (float)L.act[nt * 32 + c][16 * kt + 8 * h + j];
-                    }
-                    acc = mfma(pack8(a8), pack8(b8), acc);
-                }
-                for (int r = 0; r < 16; r++) {
-                    const int u = crow(r, h), k = nt * 32 + c;
-                    if (u < kOut) atomicAdd(&grads[oW4 + k * kOut + u], acc[r]);
-                }
-            }
-            if (lane < kOut) {
-                float sb = 0.0f;
-                for (int s = 0; s < 32; s++) sb += (float)L.dz[lane][s];
-                atomicAdd(&grads[oB4 + lane], sb);
-            }
-            __syncthreads();
-        }
-        // dA3 = W4 dZ4 -> dZ3 = dA3 * hswish'(z3)
-        f32x16 dz[2];
-        {
-            const bf16x8 b = pack8(dz4);
-            for (int mt = 0; mt < 2; mt++) {
-                f32x16 z = {};
-                z = mfma(load_frag(frags, kFragB4 + mt, lane), b, z);
-                for (int r = 0; r < 16; r++) z[r] *= hswish_grad(L.z[tile][2][mt][r][lane]);
-                dz[mt] = z;
-            }
-        }
-        // ---- layers 3, 2, 1: weight gradients from (dZ_l, a_{l-1}); propagate to l-1
-        const int wOff[3] = {oW3, oW2, oW1}, bOff[3] = {oB3, oB2, oB1}, bfrag[2] = {kFragB3, kFragB2};
-        for (int li = 0; li < 3; li++) {
-            const int layer = 2 - li;  // z index of this layer's pre-activation: 2 = layer 3
-            const int kin = layer == 0 ? kIn : kHidden;
-            // LDS: dz^T rows = units of this layer; act^T rows = inputs of this layer
-            for (int mt = 0; mt < 2; mt++)
-                for (int r = 0; r < 16; r++) L.dz[mt * 32 + crow(r, h)][c] = (__bf16)dz[mt][r];
-            if (layer > 0) {
-                for (int mt = 0; mt < 2; mt++)
-                    for (int r = 0; r < 16; r++)
-                        L.act[mt * 32 + crow(r, h)][c] = (__bf16)hswish(L.z[tile][layer - 1][mt][r][lane]);
-            } else {
-                for (int k = 0; k < kIn; k++)
-                    if (h == 0) L.act[k][c] = (__bf16)L.x[32 * tile + c][k];
-            }
-            __syncthreads();
-            // dW^T[u][k] : M = 64 units (2 m-tiles), N = kin inputs (1 or 2 n-tiles), K = 32 samples
-            for (int mt = 0; mt < 2; mt++) {
-                for (int nt = 0; nt < (kin + 31) / 32; nt++) {
-                    f32x16 acc = {};
-                    for (int kt = 0; kt < 2; kt++) {
-                        float a8[8], b8[8];
-                        for (int j = 0; j < 8; j++) {
-                            a8[j] = (float)L.dz[mt * 32 + c][16 * kt + 8 * h + j];
-                            const int k = nt * 32 + c;
-                            b8[j] = k < kin ? (float)L.act[k][16 * kt + 8 * h + j] : 0.0f;
-                        }
-                        acc = mfma(pack8(a8), pack8(b8), acc);
-                    }
-                    for (int r = 0; r < 16; r++) {
-                        const int u = mt * 32 + crow(r, h), k = nt * 32 + c;
-                        if (k < kin) atomicAdd(&grads[wOff[li] + k * kHidden + u], acc[r]);
-                    }
-                }
-            }
-            {
-                float sb = 0.0f;
-                for (int s = 0; s < 32; s++) sb += (float)L.dz[lane][s];
-                atomicAdd(&grads[bOff[li] + lane], sb);
-            }
-            __syncthreads();
-            if (layer == 0) break;
-            // dA_{l-1} = W_l dZ_l (B operand = dZ registers, k permuted), times hswish'(z_{l-1})
-            bf16x8 b[4];
-            for (int mt = 0; mt < 2; mt++) {
-                float v[16];
-                for (int r = 0; r < 16; r++) v[r] = dz[mt][r];
-                b[mt * 2 + 0] = pack8(v);
-                b[mt * 2 + 1] = pack8(v + 8);
-            }
-            for (int mt = 0; mt < 2; mt++) {
-                f32x16 z = {};
-                for (int kt = 0; kt < 4; kt++) z = mfma(load_frag(frags, bfrag[li] + mt * 4 + kt, lane), b[kt], z);
-                for (int r = 0; r < 16; r++) z[r] *= hswish_grad(L.z[tile][layer - 1][mt][r][lane]);
-                dz[mt] = z;
-            }
-        }
-    }
-    // loss: lanes of half 0 carry the per-sample terms
-    for (int off = 32; off > 0; off >>= 1) lossv += __shfl_xor(lossv, off);
-    if (lane == 0) atomicAdd(loss_acc, lossv);
 }
 
-__global__ void adam_kernel(float* params, float* grads, float* m, float* v, float lr, float b1, float b2, float eps,
-                            int t) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= kParams) return;
-    const float g = grads[i];
+// Rows: hashed draws from the n samples (`rows` = the batch) by the model's step counter plus `step`, or, with
+// no counter, samples 0 .. n - 1 (rows = n).
+// out: ATOMIC ? the gradients, with the loss at `loss` : the partial buffers, the loss at [kParams].
+template <bool ATOMIC>
+__global__ __launch_bounds__(64 * kTrainWaves, 1) void train_kernel(
+    const float* __restrict__ samples, int n, int stride, const float* __restrict__ params,
+    const float* __restrict__ stats, const uint4* __restrict__ frags, float* __restrict__ out,
+    float* __restrict__ loss, uint32_t seed, const int* __restrict__ counter, int step, int rows, float invB) {
+    __shared__ TrainLds L;
+    const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = 32 * w + c;  // this lane's row within the block
+    float mean[8], inv[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        mean[j] = stats[8 * h + j];
+        inv[j] = stats[16 + 8 * h + j];
+    }
+    const uint32_t draw = counter ? (uint32_t)(*counter + step) * 0x632BE5ABu : 0u;
+    // this lane's half of its row's features and the row's D, fetched ahead of the rows in work
+    float next[9];
+    auto fetch = [&](int b) {
+        const uint32_t row = (uint32_t)b * kTrainRows + (uint32_t)col;
+        uint32_t idx = row < (uint32_t)rows ? row : 0u;
+        if (counter) idx = hash_u32(seed ^ hash_u32(draw + row)) % (uint32_t)n;
+        const float* src = samples + (size_t)idx * stride;
+#pragma unroll
+        for (int j = 0; j < 8; j++) next[j] = src[8 * h + j];
+        next[8] = src[kIn];
+    };
+    const int blocks = (rows + kTrainRows - 1) / kTrainRows;
+    fetch(blockIdx.x);
+#pragma unroll
+    for (int k = 0; k < kFrags / kTrainWaves; k++)
+        L.frag[64 * kTrainWaves * k + threadIdx.x] = frags[64 * kTrainWaves * k + threadIdx.x];
+    if (threadIdx.x < 3 * kHidden) {
+        const int l = threadIdx.x / kHidden, u = threadIdx.x % kHidden;
+        L.bias[l][u] = params[(l == 0 ? oB1 : l == 1 ? oB2 : oB3) + u];
+    }
+    auto frag = [&](int k) { return __builtin_bit_cast(bf16x8, L.frag[64 * k + lane]); };
+    if (h == 0) L.x[kIn][col] = (__bf16)1.0f;
+    __syncthreads();
+    f32x16 acc[4] = {};
+    float lossv = 0.0f, db4[2] = {0.0f, 0.0f};
+    for (int b = blockIdx.x; b < blocks; b += gridDim.x) {
+        const bool valid = (uint32_t)b * kTrainRows + (uint32_t)col < (uint32_t)rows;
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = (next[j] - mean[j]) * inv[j];
+        const float T = __expf(-next[8]);
+        if (b + (int)gridDim.x < blocks) fetch(b + (int)gridDim.x);
+        const bf16x8 xb = pack8(x);
+#pragma unroll
+        for (int j = 0; j < 8; j++) L.x[8 * h + j][col] = xb[j];
+        // ---- forward: pre-activations z stay in registers, activations go to LDS
+        float z[3][32];
+        bf16x8 a[4];
+#pragma unroll
+        for (int l = 0; l < 3; l++) {
+            f32x16 t[2];  // accumulators start at the biases
+#pragma unroll
+            for (int r = 0; r < 32; r++) t[r / 16][r % 16] = L.bias[l][(r / 16) * 32 + crow(r % 16, h)];
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) {
+                if (l == 0) t[mt] = mfma(frag(kFragF1 + mt), xb, t[mt]);
+                else
+                    for (int kt = 0; kt < 4; kt++)
+                        t[mt] = mfma(frag((l == 1 ? kFragF2 : kFragF3) + mt * 4 + kt), a[kt], t[mt]);
+            }
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) {
+                float v[16];
+                for (int r = 0; r < 16; r++) {
+                    z[l][mt * 16 + r] = t[mt][r];
+                    v[r] = hswish(t[mt][r]);
+                }
+                a[2 * mt] = pack8(v);
+                a[2 * mt + 1] = pack8(v + 8);
+            }
+#pragma unroll
+            for (int r = 0; r < 32; r++) L.act[l][(r / 16) * 32 + crow(r % 16, h)][col] = a[r / 8][r % 8];
+        }
+        // ---- output layer, loss and dZ4 (the outputs of row c are in the lanes of half 0)
+        f32x16 o = {};
+#pragma unroll
+        for (int kt = 0; kt < 4; kt++) o = mfma(frag(kFragF4 + kt), a[kt], o);
+        float dz4[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (h == 0) {
+            const float o0 = o[0] + params[oB4], o1 = o[1] + params[oB4 + 1];
+            const float p = __expf(o0), r = p - T, ar = fabsf(r);
+            const float e = softplus(o1), sig = 1.0f / (1.0f + __expf(-o1));
+            if (valid) {
+                lossv += r * r + (e - ar) * (e - ar);
+                dz4[0] = (2.0f * r * p) * invB;
+                dz4[1] = (2.0f * (e - ar) * sig) * invB;
+            }
+        }
+        const bf16x8 d4 = pack8(dz4);
+        if (h == 0) {
+            L.dz4[0][col] = d4[0];
+            L.dz4[1][col] = d4[1];
+            db4[0] += (float)d4[0];
+            db4[1] += (float)d4[1];
+        }
+        // ---- backward: dA = W dZ (dZ in registers as the B operand, k permuted), dZ = dA hswish'(z)
+#pragma unroll
+        for (int l = 2; l >= 0; l--) {
+            f32x16 t[2] = {};
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) {
+                if (l == 2) t[mt] = mfma(frag(kFragB4 + mt), d4, t[mt]);
+                else
+                    for (int kt = 0; kt < 4; kt++)
+                        t[mt] = mfma(frag((l == 1 ? kFragB3 : kFragB2) + mt * 4 + kt), a[kt], t[mt]);
+            }
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) {
+                float v[16];
+                for (int r = 0; r < 16; r++) v[r] = t[mt][r] * hswish_grad(z[l][mt * 16 + r]);
+                a[2 * mt] = pack8(v);
+                a[2 * mt + 1] = pack8(v + 8);
+            }
+#pragma unroll
+            for (int r = 0; r < 32; r++) L.dz[l][(r / 16) * 32 + crow(r % 16, h)][col] = a[r / 8][r % 8];
+        }
+        __syncthreads();
+        // ---- weight gradients: M = units (rows of dZ^T), N = inputs (rows of a^T), K = the block's rows
+        // wave w: tile (w / 2, w % 2) of dW3 and dW2; waves 0, 1: dW1 and db1 (the inputs with their row of ones), db2;
+        // waves 2, 3: db3 (products with ones), dW4
+        const int mt = w >> 1, nt = w & 1;
+        const bool lower = w < 2;
+        const __bf16* A[4] = {L.dz[2][32 * mt + c], L.dz[1][32 * mt + c], L.dz[lower ? 0 : 2][32 * nt + c],
+                              lower ? L.dz[1][32 * nt + c] : L.dz4[c & 1]};
+        const __bf16* B[4] = {L.act[1][32 * nt + c], L.act[0][32 * nt + c], L.x[lower ? c : kIn],
+                              lower ? L.x[kIn] : L.act[2][32 * nt + c]};
+#pragma unroll
+        for (int kt = 0; kt < kTrainRows / 16; kt++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int k = 16 * kt + 8 * h;
+                acc[q] = mfma(*reinterpret_cast<const bf16x8*>(A[q] + k), *reinterpret_cast<const bf16x8*>(B[q] + k),
+                              acc[q]);
+            }
+        __syncthreads();  // the next rows overwrite the tiles
+    }
+    float* g = ATOMIC ? out : out + (size_t)blockIdx.x * kPartial;
+    // loss and output biases: summed over the wave, then over the four waves
+    for (int off = 32; off > 0; off >>= 1) {
+        lossv += __shfl_xor(lossv, off);
+        db4[0] += __shfl_xor(db4[0], off);
+        db4[1] += __shfl_xor(db4[1], off);
+    }
+    if (lane == 0) {
+        L.red[w][0] = lossv;
+        L.red[w][1] = db4[0];
+        L.red[w][2] = db4[1];
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        float s = 0.0f;
+        for (int k = 0; k < kTrainWaves; k++) s += L.red[k][threadIdx.x];
+        if (threadIdx.x == 0) put<ATOMIC>(ATOMIC ? loss : g, ATOMIC ? 0 : kParams, s);
+        else put<ATOMIC>(g, oB4 + (int)threadIdx.x - 1, s);
+    }
+    const int mt = w >> 1, nt = w & 1;
+#pragma unroll
+    for (int r = 0; r < 16; r += 4) {
+        const int u = 2 * r + 4 * h;  // crow(r, h)
+        put4<ATOMIC>(g, oW3 + (32 * nt + c) * kHidden + 32 * mt + u, acc[0], r);
+        put4<ATOMIC>(g, oW2 + (32 * nt + c) * kHidden + 32 * mt + u, acc[1], r);
+        if (w < 2) {
+            if (c < kIn) put4<ATOMIC>(g, oW1 + c * kHidden + 32 * nt + u, acc[2], r);
+            if (c == kIn) put4<ATOMIC>(g, oB1 + 32 * nt + u, acc[2], r);
+            if (c == 0) put4<ATOMIC>(g, oB2 + 32 * nt + u, acc[3], r);
+        } else if (c == 0) {
+            put4<ATOMIC>(g, oB3 + 32 * nt + u, acc[2], r);
+        }
+    }
+    if (w >= 2 && h == 0) {
+        put<ATOMIC>(g, oW4 + (32 * nt + c) * kOut, acc[3][0]);
+        put<ATOMIC>(g, oW4 + (32 * nt + c) * kOut + 1, acc[3][1]);
+    }
+}
+
+// Where parameter i enters the packed fragments (the inverse of pack_kernel's maps), written there.
+__device__ __forceinline__ void kperm_inverse(int k, int& kt, int& h, int& j) {
+    kt = (k / 32) * 2 + (k % 32) / 16;
+    h = (k / 4) % 2;
+    j = ((k % 16) / 8) * 4 + k % 4;
+}
+__device__ void scatter_param(int i, float p, uint4* frags, uint4* hfrags) {
+    __bf16* fb = reinterpret_cast<__bf16*>(frags);
+    _Float16* fh = reinterpret_cast<_Float16*>(hfrags);
+    auto slot = [](int frag, int h, int c, int j) { return (frag * 64 + h * 32 + c) * 8 + j; };
+    const float bw = bf16_value(p);
+    auto bias = [&](int frag, int u) {
+        const float hi = (float)(_Float16)p;
+        fh[slot(frag, 0, u % 32, 0)] = (_Float16)hi;
+        fh[slot(frag, 0, u % 32, 1)] = (_Float16)(p - hi);
+    };
+    int kt, h, j;
+    if (i < oB1) {
+        const int k = i / kHidden, u = i % kHidden;
+        fb[slot(kFragF1 + u / 32, k / 8, u % 32, k % 8)] = (__bf16)p;
+        fh[slot(kHF1 + 2 * (u / 32) + 1, k / 8, u % 32, k % 8)] = (_Float16)bw;
+    } else if (i < oW2) {
+        bias(kHF1 + 2 * ((i - oB1) / 32), i - oB1);
+    } else if (i < oW4) {
+        const bool two = i < oW3;
+        const int e = i - (two ? oW2 : oW3), hf = two ? kHF2 : kHF3;
+        if (e >= kHidden * kHidden) {
+            const int u = e - kHidden * kHidden;
+            bias(hf + 5 * (u / 32), u);
+        } else {
+            const int k = e / kHidden, u = e % kHidden;
+            kperm_inverse(k, kt, h, j);
+            fb[slot((two ? kFragF2 : kFragF3) + (u / 32) * 4 + kt, h, u % 32, j)] = (__bf16)p;
+            fh[slot(hf + 5 * (u / 32) + 1 + kt, h, u % 32, j)] = (_Float16)bw;
+            kperm_inverse(u, kt, h, j);
+            fb[slot((two ? kFragB2 : kFragB3) + (k / 32) * 4 + kt, h, k % 32, j)] = (__bf16)p;
+        }
+    } else if (i < oB4) {
+        const int k = (i - oW4) / kOut, o = (i - oW4) % kOut;
+        kperm_inverse(k, kt, h, j);
+        fb[slot(kFragF4 + kt, h, o, j)] = (__bf16)p;
+        fh[slot(kHF4 + kt, h, o, j)] = (_Float16)bw;
+        fb[slot(kFragB4 + k / 32, 0, k % 32, o)] = (__bf16)p;
+    }
+}
+
+// One Adam update from the workgroups' partial gradients: a block takes 64 parameters, each summed by 4
+// threads (every fourth partial) in a fixed order; the first of them updates the parameter, its moments
+// and its places in the packed fragments. Parameter kParams is the loss. One launch in place of a
+// reduction, Adam, a repack of all 4096 fragment lanes and the clearing of the gradients.
+__global__ __launch_bounds__(256) void update_kernel(const float* __restrict__ part, int nb, float* params, float* m,
+                                                     float* v, uint4* frags, uint4* hfrags, float* loss, float lr,
+                                                     float b1, float b2, float eps, const int* __restrict__ counter,
+                                                     int step) {
+    __shared__ float sum[4][64];
+    const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+    float s = 0.0f;
+    if (i <= kParams) {
+#pragma unroll 8
+        for (int b = grp; b < nb; b += 4) s += part[(size_t)b * kPartial + i];
+    }
+    sum[grp][lane] = s;
+    __syncthreads();
+    if (grp != 0 || i > kParams) return;
+    const float g = (sum[0][lane] + sum[1][lane]) + (sum[2][lane] + sum[3][lane]);
+    if (i == kParams) {
+        *loss = g;
+        return;
+    }
+    const int t = *counter + step + 1;
     const float mi = b1 * m[i] + (1.0f - b1) * g;
     const float vi = b2 * v[i] + (1.0f - b2) * g * g;
     m[i] = mi;
     v[i] = vi;
     const float mh = mi / (1.0f - powf(b1, (float)t)), vh = vi / (1.0f - powf(b2, (float)t));
-    params[i] -= lr * mh / (sqrtf(vh) + eps);
-    grads[i] = 0.0f;
+    const float p = params[i] - lr * mh / (sqrtf(vh) + eps);
+    params[i] = p;
+    scatter_param(i, p, frags, hfrags);
 }
+
+__global__ void advance_kernel(int* counter, int steps) { *counter += steps; }
 
 __global__ void zero_kernel(float* p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -405,24 +523,22 @@ int surrogate_train(void* model, const float* samples, int n, int stride, int ba
                     uint32_t seed, float* loss_out, void* stream) {
     hipStream_t s = (hipStream_t)stream;
     ModelPtrs p = ptrs(model);
-    float* step_counter = p.stats + 32;
-    int t0 = 0;
-    if (hipMemcpyAsync(&t0, step_counter, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess) return MM_E_DEVICE;
-    if (hipStreamSynchronize(s) != hipSuccess) return MM_E_DEVICE;
-    const int waves = batch / 64;
+    int* counter = reinterpret_cast<int*>(p.stats + 32);  // Adam steps taken; stays on the device
+    const int nb = std::min(kMaxTrainBlocks, (batch + kTrainRows - 1) / kTrainRows);
+    float* part = nullptr;  // the workgroups' partial gradients, for this call
+    if (steps > 0 && hipMallocAsync((void**)&part, sizeof(float) * (size_t)nb * kPartial, s) != hipSuccess)
+        return MM_E_DEVICE;
     for (int i = 0; i < steps; i++) {
-        float* lacc = loss_out ? loss_out + i : p.stats + 33;
-        hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, s, lacc, 1);
-        hipLaunchKernelGGL(train_kernel, dim3(waves), dim3(64), 0, s, samples, n, stride, p.params, p.stats, p.frags,
-                           p.grads, lacc, seed, t0 + i, 0, 1.0f / (float)batch);
-        hipLaunchKernelGGL(adam_kernel, dim3(blocks(kParams, 256)), dim3(256), 0, s, p.params, p.grads, p.m, p.v, lr,
-                           0.9f, 0.999f, 1e-8f, t0 + i + 1);
-        hipLaunchKernelGGL(pack_kernel, dim3(blocks(kPackThreads, 256)), dim3(256), 0, s, p.params, p.frags, p.hfrags);
+        hipLaunchKernelGGL(train_kernel<false>, dim3(nb), dim3(64 * kTrainWaves), 0, s, samples, n, stride, p.params,
+                           p.stats, p.frags, part, nullptr, seed, counter, i, batch, 1.0f / (float)batch);
+        hipLaunchKernelGGL(update_kernel, dim3(blocks(kParams + 1, 64)), dim3(256), 0, s, part, nb, p.params, p.m, p.v,
+                           p.frags, p.hfrags, loss_out ? loss_out + i : p.stats + 33, lr, 0.9f, 0.999f, 1e-8f, counter,
+                           i);
     }
-    int t1 = t0 + steps;
-    if (hipMemcpyAsync(step_counter, &t1, sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess) return MM_E_DEVICE;
-    if (hipStreamSynchronize(s) != hipSuccess) return MM_E_DEVICE;
-    return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
+    hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(1), 0, s, counter, steps);
+    const int e = hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
+    if (part) (void)hipFreeAsync(part, s);
+    return hipStreamSynchronize(s) == hipSuccess ? e : MM_E_DEVICE;
 }
 
 int surrogate_load(void* model, const float* params, const float* stats, void* stream) {
@@ -442,8 +558,9 @@ int surrogate_gradient(const void* model, const float* samples, int n, int strid
     ModelPtrs p = ptrs(const_cast<void*>(model));
     hipLaunchKernelGGL(zero_kernel, dim3(blocks(kParams, 256)), dim3(256), 0, s, grad_out, kParams);
     hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, s, loss_out, 1);
-    hipLaunchKernelGGL(train_kernel, dim3(blocks(n, 64)), dim3(64), 0, s, samples, n, stride, p.params, p.stats, p.frags,
-                       grad_out, loss_out, 0u, 0, 1, 1.0f / (float)n);
+    const unsigned nb = std::min(blocks(n, kTrainRows), (unsigned)kMaxTrainBlocks);
+    hipLaunchKernelGGL(train_kernel<true>, dim3(nb), dim3(64 * kTrainWaves), 0, s, samples, n, stride, p.params,
+                       p.stats, p.frags, grad_out, loss_out, 0u, nullptr, 0, n, 1.0f / (float)n);
     return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
 }
 

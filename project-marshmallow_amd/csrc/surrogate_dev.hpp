@@ -43,14 +43,10 @@ __host__ __device__ inline int crow(int r, int h) { return 8 * (r / 4) + 4 * h +
 __device__ __forceinline__ float hswish(float z) {
     return z * __builtin_amdgcn_fmed3f(__builtin_fmaf(z, 1.0f / 6.0f, 0.5f), 0.0f, 1.0f);
 }
-// d hswish / dz: 0 below -3, 1 above 3, z / 3 + 1/2 between
+// d hswish / dz: 0 below -3, 1 above 3, z / 3 + 1/2 between (one compare: outside, z clamped to [0, 1] is the value)
 __device__ __forceinline__ float hswish_grad(float z) {
-    return z <= -3.0f ? 0.0f : (z >= 3.0f ? 1.0f : __builtin_fmaf(z, 1.0f / 3.0f, 0.5f));
-}
-
-__device__ __forceinline__ bf16x8 load_frag(const uint4* frags, int frag, int lane) {
-    uint4 u = frags[frag * 64 + lane];
-    return __builtin_bit_cast(bf16x8, u);
+    const float out = __builtin_amdgcn_fmed3f(z, 0.0f, 1.0f), in = __builtin_fmaf(z, 1.0f / 3.0f, 0.5f);
+    return fabsf(z) >= 3.0f ? out : in;
 }
 
 __device__ __forceinline__ bf16x8 pack8(const float* v) {
@@ -63,53 +59,10 @@ __device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// Forward pass of one 32-sample tile. `xb` is the B operand of layer 1 (this lane's 8 input
-// features of sample lane % 32: features 8h..8h+7, already normalised). Writes the pre-activations
-// of the three hidden layers when `zsave` is non-null (16 floats per m-tile per layer per lane) and
-// returns the two outputs of sample lane % 32 in lanes of half 0 (rows 0 and 1 of the last tile).
+// Outputs of one sample.
 struct FwdOut {
     float o0, o1;
 };
-
-__device__ __forceinline__ FwdOut mlp_forward_tile(const uint4* __restrict__ frags, const float* __restrict__ params,
-                                                   bf16x8 xb, float* zsave /* [3][2][16] or null */) {
-    const int lane = threadIdx.x & 63, h = lane >> 5;
-    // layer 1: K = 16 (natural feature order)
-    f32x16 acc[2];
-    for (int mt = 0; mt < 2; mt++) {
-        f32x16 z = {};
-        acc[mt] = mfma(load_frag(frags, kFragF1 + mt, lane), xb, z);
-    }
-    bf16x8 b[4];
-    const int bias[3] = {oB1, oB2, oB3};
-    const int ffrag[2] = {kFragF2, kFragF3};
-    for (int layer = 0; layer < 3; layer++) {
-        // bias + activation, repack as the next layer's B operand (8 consecutive accumulators = one k-step)
-        for (int mt = 0; mt < 2; mt++) {
-            float v[16];
-            for (int r = 0; r < 16; r++) {
-                float zz = acc[mt][r] + params[bias[layer] + mt * 32 + crow(r, h)];
-                if (zsave) zsave[(layer * 2 + mt) * 16 + r] = zz;
-                v[r] = hswish(zz);
-            }
-            b[mt * 2 + 0] = pack8(v);
-            b[mt * 2 + 1] = pack8(v + 8);
-        }
-        if (layer == 2) break;
-        for (int mt = 0; mt < 2; mt++) {
-            f32x16 z = {};
-            for (int kt = 0; kt < 4; kt++) z = mfma(load_frag(frags, ffrag[layer] + mt * 4 + kt, lane), b[kt], z);
-            acc[mt] = z;
-        }
-    }
-    // output layer: 1 m-tile (rows 0, 1 used), K = 64
-    f32x16 o = {};
-    for (int kt = 0; kt < 4; kt++) o = mfma(load_frag(frags, kFragF4 + kt, lane), b[kt], o);
-    FwdOut r;
-    r.o0 = o[0] + params[oB4 + 0];  // row crow(0, 0) = 0 in lanes of half 0
-    r.o1 = o[1] + params[oB4 + 1];  // row 1
-    return r;
-}
 
 // A wave-uniform pointer made explicit (scalar registers), whatever the optimiser could prove.
 template <class T>
