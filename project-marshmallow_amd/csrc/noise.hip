@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 #include <float.h>
+#include <algorithm>
 #include <mutex>
 #include "mm_internal.hpp"
 #include "cr_math.hpp"
@@ -209,10 +210,9 @@ __device__ __forceinline__ void hash3(uint32_t x, uint32_t y, uint32_t z, uint32
     a = v0; b = v1; c = v2;
 }
 __device__ __forceinline__ float u01(uint32_t h) { return (float)(h >> 8) * (1.0f / 16777216.0f); }
-__device__ __forceinline__ int wrapi(int i, int n) {
-    int r = i % n;
-    return r < 0 ? r + n : r;
-}
+// i modulo n, n a power of two as every lattice period here is (4 << octaves): one AND, where the remainder by a
+// run-time divisor takes about 25 instructions, three times per hash.
+__device__ __forceinline__ int wrapi(int i, int n) { return i & (n - 1); }
 __device__ __forceinline__ float clamp01(float v) { return v < 0.f ? 0.f : (v > 1.f ? 1.f : v); }
 __device__ __forceinline__ float lerp_(float a, float b, float t) { return a + t * (b - a); }
 __device__ __forceinline__ uint32_t layer_seed(uint32_t seed, uint32_t layer) {
@@ -244,6 +244,9 @@ struct LdsCells {
         uy = v.y;
         uz = v.z;
     }
+    __device__ __forceinline__ const float4* at(int x, int y, int z) const {
+        return cell + (((z - bz) * ny + (y - by)) * nx + (x - bx));
+    }
 };
 
 // Inverted F1 cellular noise on a periodic grid of `cells`^3 cells.
@@ -274,15 +277,31 @@ __device__ __forceinline__ float worley_at(float px, float py, float pz, int cel
     return 1.0f - (d < 1.0f ? d : 1.0f);
 }
 
-__device__ float worley(float px, float py, float pz, int cells, uint32_t seed) {
-    return worley_at(px, py, pz, cells, HashCells{cells, seed});
-}
-
-__device__ float worley_fbm(float px, float py, float pz, int cells, uint32_t seed) {
-    float a = worley(px, py, pz, cells, seed);
-    float b = worley(px, py, pz, cells * 2, seed + 1u);
-    float c = worley(px, py, pz, cells * 4, seed + 2u);
-    return (0.625f * a + 0.25f * b) + 0.125f * c;
+// worley_at over staged cells: the same arithmetic, each row of neighbours at constant offsets from its first.
+__device__ __forceinline__ float worley_at(float px, float py, float pz, int cells, const LdsCells& src) {
+    const float qx = px * (float)cells, qy = py * (float)cells, qz = pz * (float)cells;
+    const int ix = (int)floorf(qx), iy = (int)floorf(qy), iz = (int)floorf(qz);
+    const float4* home = src.at(ix - 1, iy, iz);
+    float bx[3], best = 1e30f;
+#pragma unroll
+    for (int o = 0; o < 3; o++) bx[o] = qx - (float)(ix + o - 1);
+#pragma unroll
+    for (int oz = -1; oz <= 1; oz++) {
+        const float bz = qz - (float)(iz + oz);
+#pragma unroll
+        for (int oy = -1; oy <= 1; oy++) {
+            const float by = qy - (float)(iy + oy);
+            const float4* row = home + (oz * src.ny + oy) * src.nx;
+#pragma unroll
+            for (int o = 0; o < 3; o++) {
+                const float4 u = row[o];
+                const float dx = bx[o] - u.x, dy = by - u.y, dz = bz - u.z;
+                best = __builtin_fminf(((dx * dx) + (dy * dy)) + (dz * dz), best);
+            }
+        }
+    }
+    const float d = sqrt_rn(best);
+    return 1.0f - (d < 1.0f ? d : 1.0f);
 }
 
 __constant__ float kGrad[12][3] = {{1, 1, 0}, {-1, 1, 0}, {1, -1, 0}, {-1, -1, 0}, {1, 0, 1},  {-1, 0, 1},
@@ -324,19 +343,6 @@ __device__ __forceinline__ float perlin_at(float px, float py, float pz, int per
     float x01 = lerp_(n[4], n[5], ux), x11 = lerp_(n[6], n[7], ux);
     float y0 = lerp_(x00, x10, uy), y1 = lerp_(x01, x11, uy);
     return lerp_(y0, y1, uz);
-}
-
-__device__ float perlin_tiled(float px, float py, float pz, int period, uint32_t seed) {
-    return perlin_at(px, py, pz, period, HashGrads{period, seed});
-}
-
-__device__ float perlin_fbm(float px, float py, float pz, int period, uint32_t seed) {
-    float s = 0.f, w = 1.f;
-    for (int o = 0; o < 4; o++) {
-        s = s + w * perlin_tiled(px, py, pz, period << o, seed + (uint32_t)o);
-        w = w * 0.5f;
-    }
-    return s * (1.0f / 1.875f);
 }
 
 __device__ float value2(float px, float py, int period, uint32_t seed) {
@@ -408,153 +414,53 @@ __device__ __forceinline__ uint32_t low_level_seed(uint32_t seed, int l) {
     return l < 4 ? layer_seed(seed, 1) + (uint32_t)l : layer_seed(seed, 2 + (uint32_t)(l - 4) / 3) + (uint32_t)((l - 4) % 3);
 }
 
-// Bricks of the low-res kernel (texels per axis) and the lattice cells a block can stage in LDS.
+// ---- hi-res volume: 3 Worley layers of 3 octaves (cells 4..64); level l is layer l / 3, octave l % 3.
+constexpr int kHiLevels = 9;
+__host__ __device__ constexpr int hi_level_cells(int l) { return (4 << (l / 3)) << (l % 3); }
+__device__ __forceinline__ uint32_t hi_level_seed(uint32_t seed, int l) {
+    return layer_seed(seed, 6 + (uint32_t)l / 3) + (uint32_t)l % 3;
+}
+
+// Bricks of the volume kernels (texels per axis, 256 work-items each) and the lattice cells a block may stage
+// in LDS at a time (53 KB: three blocks a CU).
 constexpr int kBrickX = 8, kBrickY = 8, kBrickZ = 4;
-constexpr int kStageCap = 1536;  // staged cells per block: 24 KB of LDS
+constexpr int kStageCap = 3376;
+// A level is staged when its box has fewer cells than the brick's texels would hash between them.
+constexpr int kStageLevelCap = 27 * kBrickX * kBrickY * kBrickZ / 2;
 
-// Sources of the low-res levels: get<l>() hands out the lattice data of level l.
-struct LowResHash {
-    uint32_t seed;
-    template <int L>
-    __device__ __forceinline__ auto get() const {
-        if constexpr (L < 4) return HashGrads{low_level_cells(L), low_level_seed(seed, L)};
-        else return HashCells{low_level_cells(L), low_level_seed(seed, L)};
-    }
-};
-
-// Lattice cells of one level staged for a brick: cells [b, b + n) per axis, at offset `off`.
+// Lattice cells of one level around a brick: cells [b, b + n) per axis, staged at offset `off` (-1: not staged).
 struct StageMeta {
     int bx, by, bz, nx, ny, nz, off;
 };
 
-struct LowResLds {
-    const float4* cells;
-    const StageMeta* meta;
-    __device__ __forceinline__ LdsCells level(int l) const {
-        const StageMeta& m = meta[l];
-        return LdsCells{cells + m.off, m.bx, m.by, m.bz, m.nx, m.ny};
-    }
-    template <int L>
-    __device__ __forceinline__ LdsCells get() const { return level(L); }
-};
-
-// The staged boxes of a 128^3 volume. Bricks start at multiples of 8 (x, y) and 4 (z), and texel t
-// sits at q = (2t + 1) c / 256 in cell units (exact), so a brick of B texels spans
-// floor(q1) - floor(q0) = max(B c / 128 - 1, 0) cells at every position: the boxes that axis_span
-// computes have the same size for every brick, kDim128N cells per axis (pad 1 for Worley levels).
-constexpr int kDim128Span(int l, int b) { return b * low_level_cells(l) / 128 >= 1 ? b * low_level_cells(l) / 128 - 1 : 0; }
-constexpr int kDim128N(int l, int b) { return kDim128Span(l, b) + 2 + (l < 4 ? 0 : 1); }
-constexpr int kDim128Cells(int l) { return kDim128N(l, kBrickX) * kDim128N(l, kBrickY) * kDim128N(l, kBrickZ); }
-constexpr int kDim128Off(int l) { return l == 0 ? 0 : kDim128Off(l - 1) + kDim128Cells(l - 1); }
-static_assert(kDim128N(15, 8) == 10 && kDim128N(15, 4) == 6 && kDim128N(0, 8) == 2, "128^3 staged box sizes");
-static_assert(kDim128Off(kLowLevels) <= kStageCap, "a 128^3 brick's lattice cells fit the stage");
-
-// LDS cells with a compile-time box: the 27 neighbour reads of a Worley evaluation become one base
-// address plus immediate offsets.
-template <int NX, int NY>
-struct LdsCellsC {
-    const float4* cell;
-    int bx, by, bz;
-    __device__ __forceinline__ void point(int x, int y, int z, float& ux, float& uy, float& uz) const {
-        const float4 v = cell[((z - bz) * NY + (y - by)) * NX + (x - bx)];
-        ux = v.x;
-        uy = v.y;
-        uz = v.z;
-    }
-    __device__ __forceinline__ const float4* home(int x, int y, int z) const {
-        return cell + (((z - bz) * NY + (y - by)) * NX + (x - bx));
-    }
-};
-
-// worley_at for a compile-time box: the same arithmetic, the neighbour cells read at constant
-// offsets from the home cell.
-template <int NX, int NY>
-__device__ __forceinline__ float worley_at(float px, float py, float pz, int cells, const LdsCellsC<NX, NY>& src) {
-    float qx = px * (float)cells, qy = py * (float)cells, qz = pz * (float)cells;
-    int ix = (int)floorf(qx), iy = (int)floorf(qy), iz = (int)floorf(qz);
-    const float4* h = src.home(ix, iy, iz);
-    float best = 1e30f;
-#pragma unroll
-    for (int oz = -1; oz <= 1; oz++) {
-        const float bz = qz - (float)(iz + oz);
-#pragma unroll
-        for (int oy = -1; oy <= 1; oy++) {
-            const float by = qy - (float)(iy + oy);
-#pragma unroll
-            for (int ox = -1; ox <= 1; ox++) {
-                const float4 u = h[(oz * NY + oy) * NX + ox];
-                float dx = (qx - (float)(ix + ox)) - u.x;
-                float dy = by - u.y;
-                float dz = bz - u.z;
-                float d2 = ((dx * dx) + (dy * dy)) + (dz * dz);
-                best = __builtin_fminf(d2, best);
-            }
-        }
-    }
-    float d = sqrt_rn(best);
-    return 1.0f - (d < 1.0f ? d : 1.0f);
+// The low-res texel's 32-bit word (RGBA8 or FP8 x 4).
+__device__ __forceinline__ uint32_t encode_low_res(const GenArgs& a, const float v[4]) {
+    if (a.fmt == MM_FMT_RGBA8) return q8(v[0]) | (q8(v[1]) << 8) | (q8(v[2]) << 16) | (q8(v[3]) << 24);
+    uint32_t r = 0;  // MM_FMT_FP8X4
+#pragma unroll 1
+    for (int k = 0; k < 4; k++) r |= fp8_e4m3((k < 2 ? (k == 0 ? v[0] : v[1]) : (k == 2 ? v[2] : v[3])) * a.inv_scale[k]) << (8 * k);
+    return r;
 }
 
-struct LowResLds128 {
-    const float4* cells;
-    const StageMeta* meta;
-    template <int L>
-    __device__ __forceinline__ LdsCellsC<kDim128N(L, kBrickX), kDim128N(L, kBrickY)> get() const {
-        // wave-uniform box origin (the brick's), in scalar registers
-        const int bx = __builtin_amdgcn_readfirstlane(meta[L].bx), by = __builtin_amdgcn_readfirstlane(meta[L].by),
-                  bz = __builtin_amdgcn_readfirstlane(meta[L].bz);
-        constexpr int off = kDim128Off(L);  // evaluated here, not by a device-side recursive call
-        return {cells + off, bx, by, bz};
-    }
-};
-
-template <int LY, class Src>
-__device__ __forceinline__ float worley_fbm_at(float px, float py, float pz, const Src& src) {
-    constexpr int cells = 4 << LY;
-    float a = worley_at(px, py, pz, cells, src.template get<4 + 3 * LY>());
-    float b = worley_at(px, py, pz, cells * 2, src.template get<5 + 3 * LY>());
-    float c = worley_at(px, py, pz, cells * 4, src.template get<6 + 3 * LY>());
-    return (0.625f * a + 0.25f * b) + 0.125f * c;
-}
-
-// The four channels of the low-res texel at (px, py, pz): Perlin-Worley, then Worley FBMs of
-// base frequency 8, 16 and 32.
-template <class Src>
-__device__ __forceinline__ void low_res_values(float px, float py, float pz, const Src& src, float v[4]) {
-    float s = 0.f, w = 1.f;
-    s = s + w * perlin_at(px, py, pz, 4, src.template get<0>());
-    w = w * 0.5f;
-    s = s + w * perlin_at(px, py, pz, 8, src.template get<1>());
-    w = w * 0.5f;
-    s = s + w * perlin_at(px, py, pz, 16, src.template get<2>());
-    w = w * 0.5f;
-    s = s + w * perlin_at(px, py, pz, 32, src.template get<3>());
-    const float perlin = s * (1.0f / 1.875f);
-    float p01 = clamp01(0.5f + 1.5f * perlin);
-    float wf = worley_fbm_at<0>(px, py, pz, src);
-    float pw = (p01 - (wf - 1.0f)) / (1.0f - (wf - 1.0f));
-    v[0] = clamp01(0.8f * pw - 0.04f);
-    v[1] = clamp01(0.26f + 0.9f * worley_fbm_at<1>(px, py, pz, src));
-    v[2] = clamp01(0.26f + 0.9f * worley_fbm_at<2>(px, py, pz, src));
-    v[3] = clamp01(0.26f + 0.9f * worley_fbm_at<3>(px, py, pz, src));
-}
-
-__device__ __forceinline__ void store_low_res(const GenArgs& a, long i, const float v[4]) {
+__device__ __forceinline__ void store_hi_res(const GenArgs& a, long i, const float v[3]) {
     if (a.fmt == MM_FMT_RGBA8) {
-        reinterpret_cast<uint32_t*>(a.dst)[i] = q8(v[0]) | (q8(v[1]) << 8) | (q8(v[2]) << 16) | (q8(v[3]) << 24);
-    } else {  // MM_FMT_FP8X4
-        uint32_t r = 0;
-        for (int k = 0; k < 4; k++) r |= fp8_e4m3(v[k] * a.inv_scale[k]) << (8 * k);
-        reinterpret_cast<uint32_t*>(a.dst)[i] = r;
+        reinterpret_cast<uint32_t*>(a.dst)[i] = q8(v[0]) | (q8(v[1]) << 8) | (q8(v[2]) << 16);
+    } else {  // MM_FMT_FP16X4
+        uint2 o;
+        o.x = half_bits(v[0]) | (half_bits(v[1]) << 16);
+        o.y = half_bits(v[2]);
+        reinterpret_cast<uint2*>(a.dst)[i] = o;
     }
 }
 
-// Brick kernel: a block of 256 work-items takes an 8 x 8 x 4 brick of logical texels. The lattice
-// cells the brick's texels touch at each level (about 1.2k cells for a 128^3 volume, against 356
-// hashes per texel) are hashed once into LDS; the texels then read them there. When a brick
-// touches more cells than LDS holds (small volumes, where cells outnumber texels) it hashes in
-// place. Texels whose coordinate is below the apron width are also written to the apron copy
-// (x + dim, ...).
+__device__ __forceinline__ float worley_mix(float a, float b, float c) { return (0.625f * a + 0.25f * b) + 0.125f * c; }
+// A Worley channel of the textures, and the low-res Perlin-Worley one.
+__device__ __forceinline__ float worley_channel(float wf) { return clamp01(0.26f + 0.9f * wf); }
+__device__ __forceinline__ float perlin_worley_channel(float perlin, float wf) {
+    const float p01 = clamp01(0.5f + 1.5f * perlin);
+    const float pw = (p01 - (wf - 1.0f)) / (1.0f - (wf - 1.0f));
+    return clamp01(0.8f * pw - 0.04f);
+}
 
 // Cells [floor(q(t0)) - pad, floor(q(t1)) + 1] of one axis, q(t) = ((2t + 1) / (2 dim)) * cells,
 // evaluated as the texel evaluates it (q is monotone in t, so every texel's cells lie inside).
@@ -565,65 +471,111 @@ __device__ __forceinline__ void axis_span(int t0, int t1, float inv, int cells, 
     n = ((int)floorf(q1) + 1) - base + 1;
 }
 
-// DIM128: the volume is 128^3 (asserted by the host), whose staged boxes have compile-time sizes.
-template <bool DIM128>
-__global__ __launch_bounds__(256) void low_res_brick_kernel(GenArgs a) {
-    __shared__ float4 cells[kStageCap];
-    __shared__ StageMeta meta[kLowLevels];
-    __shared__ int total;
+// Cells of a level's box around a brick of `b` texels per axis, at most (for the host's LDS size).
+inline long box_bound(int b, int dim, int cells, int pad) { return ((long)(b - 1) * cells + dim - 1) / dim + 3 + pad; }
+
+// Volumes of any size: a block of 256 work-items takes an 8 x 8 x 4 brick of logical texels, one each. The
+// lattice cells the brick's texels touch are hashed once into LDS, layer by layer (the Perlin octaves, then
+// each Worley layer's three), while a layer's levels fit `cap` cells and are fewer than half of what the texels
+// would hash; the others (small volumes at high frequencies, where cells outnumber texels) hash in place.
+// Staging layer by layer, not all levels at once, lets three to eight blocks share a CU: 72^3 low-res 120 us ->
+// 85, 32^3 hi-res 20 -> 15. Vector operations bound it (27 distances, 9 operations each, at each Worley level).
+// Texels whose coordinate is below the apron width are also written to the apron copy (x + dim, ...).
+template <bool HI>
+__global__ __launch_bounds__(256) void volume_brick_kernel(GenArgs a, int cap) {
+    extern __shared__ float4 cells[];
+    constexpr int kFirstWorley = HI ? 0 : 4;
+    __shared__ StageMeta meta[4];
     const int tid = threadIdx.x;
     const int nbx = (a.dim + kBrickX - 1) / kBrickX, nby = (a.dim + kBrickY - 1) / kBrickY;
     const int x0 = (int)(blockIdx.x % nbx) * kBrickX, y0 = (int)((blockIdx.x / nbx) % nby) * kBrickY;
     const int z0 = (int)(blockIdx.x / (nbx * nby)) * kBrickZ;
     const int x1 = min(x0 + kBrickX, a.dim) - 1, y1 = min(y0 + kBrickY, a.dim) - 1, z1 = min(z0 + kBrickZ, a.dim) - 1;
     const float inv = 1.0f / (float)(2 * a.dim);
-    if (tid < kLowLevels) {
-        const int cells = low_level_cells(tid), pad = tid < 4 ? 0 : 1;
-        StageMeta m;
-        axis_span(x0, x1, inv, cells, pad, m.bx, m.nx);
-        axis_span(y0, y1, inv, cells, pad, m.by, m.ny);
-        axis_span(z0, z1, inv, cells, pad, m.bz, m.nz);
-        m.off = m.nx * m.ny * m.nz;  // count for now; prefix-summed below
-        meta[tid] = m;
-    }
-    __syncthreads();
-    if (tid == 0) {
+    auto level_cells = [](int l) { return HI ? hi_level_cells(l) : low_level_cells(l); };
+    auto level_seed = [&](int l) { return HI ? hi_level_seed(a.seed, l) : low_level_seed(a.seed, l); };
+    // Stages levels l0 .. l0 + n - 1 (every work-item takes part).
+    auto stage = [&](int l0, int n) {
+        __syncthreads();  // the last layer's cells are no longer read
+        if (tid < n) {
+            const int l = l0 + tid, c = level_cells(l), pad = l < kFirstWorley ? 0 : 1;
+            StageMeta m;
+            axis_span(x0, x1, inv, c, pad, m.bx, m.nx);
+            axis_span(y0, y1, inv, c, pad, m.by, m.ny);
+            axis_span(z0, z1, inv, c, pad, m.bz, m.nz);
+            m.off = 0;
+            meta[tid] = m;
+        }
+        __syncthreads();
         int off = 0;
-        for (int l = 0; l < kLowLevels; l++) {
-            const int cnt = meta[l].off;
-            meta[l].off = off;
+        for (int k = 0; k < n; k++) {
+            const StageMeta m = meta[k];
+            const int cnt = m.nx * m.ny * m.nz, l = l0 + k, c = level_cells(l);
+            const bool fits = cnt <= kStageLevelCap && off + cnt <= cap;  // uniform across the block
+            if (tid == 0) meta[k].off = fits ? off : -1;
+            if (!fits) continue;
+            const uint32_t seed = level_seed(l);
+            // e / n by a reciprocal: e + 1/2 is at least 1 / (2 n) from a multiple, far beyond its rounding
+            const float rx = 1.0f / (float)m.nx, ry = 1.0f / (float)m.ny;
+            for (int e = (tid + 64 * k) & 255; e < cnt; e += 256) {
+                const int yz = (int)(((float)e + 0.5f) * rx), jx = e - yz * m.nx;
+                const int jz = (int)(((float)yz + 0.5f) * ry), jy = yz - jz * m.ny;
+                float u0, u1, u2;
+                if (l < kFirstWorley) HashGrads{c, seed}.point(m.bx + jx, m.by + jy, m.bz + jz, u0, u1, u2);
+                else HashCells{c, seed}.point(m.bx + jx, m.by + jy, m.bz + jz, u0, u1, u2);
+                cells[off + e] = make_float4(u0, u1, u2, 0.0f);
+            }
             off += cnt;
         }
-        total = off;
-    }
-    __syncthreads();
-    const int nst = total;
-    const bool staged = DIM128 || nst <= kStageCap;  // uniform across the block
-    if (staged) {
-        for (int e = tid; e < nst; e += 256) {
-            int l = 0;
-            while (l + 1 < kLowLevels && meta[l + 1].off <= e) l++;
-            const StageMeta m = meta[l];
-            const int r = e - m.off, jx = r % m.nx, jy = (r / m.nx) % m.ny, jz = r / (m.nx * m.ny);
-            float u0, u1, u2;
-            if (l < 4)
-                HashGrads{low_level_cells(l), low_level_seed(a.seed, l)}.point(m.bx + jx, m.by + jy, m.bz + jz, u0, u1, u2);
-            else
-                HashCells{low_level_cells(l), low_level_seed(a.seed, l)}.point(m.bx + jx, m.by + jy, m.bz + jz, u0, u1, u2);
-            cells[e] = make_float4(u0, u1, u2, 0.0f);
-        }
-    }
-    __syncthreads();
+        __syncthreads();
+    };
     const int x = x0 + (tid & (kBrickX - 1)), y = y0 + ((tid / kBrickX) & (kBrickY - 1)), z = z0 + tid / (kBrickX * kBrickY);
-    if (x > x1 || y > y1 || z > z1) return;
+    const bool in = x <= x1 && y <= y1 && z <= z1;
     const float px = (float)(2 * x + 1) * inv, py = (float)(2 * y + 1) * inv, pz = (float)(2 * z + 1) * inv;
-    float v[4];
-    if constexpr (DIM128)
-        low_res_values(px, py, pz, LowResLds128{cells, meta}, v);
-    else if (staged)
-        low_res_values(px, py, pz, LowResLds{cells, meta}, v);
-    else
-        low_res_values(px, py, pz, LowResHash{a.seed}, v);
+    auto lds = [&](int k) {
+        const StageMeta& m = meta[k];
+        return LdsCells{cells + m.off, m.bx, m.by, m.bz, m.nx, m.ny};
+    };
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float perlin = 0.0f;
+    if constexpr (!HI) {
+        stage(0, 4);
+        if (in) {
+            float w = 1.0f;
+#pragma unroll 1
+            for (int l = 0; l < 4; l++) {
+                const int c = level_cells(l);
+                perlin = perlin + w * (meta[l].off >= 0 ? perlin_at(px, py, pz, c, lds(l))
+                                                        : perlin_at(px, py, pz, c, HashGrads{c, level_seed(l)}));
+                w = w * 0.5f;
+            }
+        }
+        perlin = perlin * (1.0f / 1.875f);
+    }
+#pragma unroll 1
+    for (int ly = 0; ly < (HI ? 3 : 4); ly++) {
+        const int l0 = kFirstWorley + 3 * ly;
+        stage(l0, 3);
+        if (!in) continue;
+        float f[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int o = 0; o < 3; o++) {
+            const int c = level_cells(l0 + o);
+            const float w = meta[o].off >= 0 ? worley_at(px, py, pz, c, lds(o))
+                                             : worley_at(px, py, pz, c, HashCells{c, level_seed(l0 + o)});
+            f[0] = o == 0 ? w : f[0];
+            f[1] = o == 1 ? w : f[1];
+            f[2] = o == 2 ? w : f[2];
+        }
+        const float wf = worley_mix(f[0], f[1], f[2]);
+        const float ch = !HI && ly == 0 ? perlin_worley_channel(perlin, wf) : worley_channel(wf);
+        v[0] = ly == 0 ? ch : v[0];
+        v[1] = ly == 1 ? ch : v[1];
+        v[2] = ly == 2 ? ch : v[2];
+        v[3] = ly == 3 ? ch : v[3];
+    }
+    if (!in) return;
+    const uint32_t word = HI ? 0u : encode_low_res(a, v);
     const long sd = a.dim + a.apron;
     for (int cz = 0; cz < 2; cz++) {
         const int zs = z + cz * a.dim;
@@ -634,31 +586,180 @@ __global__ __launch_bounds__(256) void low_res_brick_kernel(GenArgs a) {
             for (int cx = 0; cx < 2; cx++) {
                 const int xs = x + cx * a.dim;
                 if (cx && xs >= sd) break;
-                store_low_res(a, ((long)zs * sd + ys) * sd + xs, v);
+                const long i = ((long)zs * sd + ys) * sd + xs;
+                if constexpr (HI) store_hi_res(a, i, v);
+                else reinterpret_cast<uint32_t*>(a.dst)[i] = word;
             }
         }
     }
 }
 
-__global__ __launch_bounds__(256) void hi_res_kernel(GenArgs a) {
-    const int sd = a.dim + a.apron;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= sd * sd * sd) return;
-    const int x = (i % sd) % a.dim, y = ((i / sd) % sd) % a.dim, z = (i / (sd * sd)) % a.dim;
-    const float inv = 1.0f / (float)(2 * a.dim);
-    float px = (float)(2 * x + 1) * inv, py = (float)(2 * y + 1) * inv, pz = (float)(2 * z + 1) * inv;
-    float v[3];
-    v[0] = clamp01(0.26f + 0.9f * worley_fbm(px, py, pz, 4, layer_seed(a.seed, 6)));
-    v[1] = clamp01(0.26f + 0.9f * worley_fbm(px, py, pz, 8, layer_seed(a.seed, 7)));
-    v[2] = clamp01(0.26f + 0.9f * worley_fbm(px, py, pz, 16, layer_seed(a.seed, 8)));
-    if (a.fmt == MM_FMT_RGBA8) {
-        reinterpret_cast<uint32_t*>(a.dst)[i] = q8(v[0]) | (q8(v[1]) << 8) | (q8(v[2]) << 16);
-    } else {  // MM_FMT_FP16X4
-        uint2 o;
-        o.x = half_bits(v[0]) | (half_bits(v[1]) << 16);
-        o.y = half_bits(v[2]);
-        reinterpret_cast<uint2*>(a.dst)[i] = o;
+// ---- the 128^3 low-res volume (the configured size). Bricks of 16 x 8 x 8 texels start at multiples of their
+// size, and texel t sits at q = (2t + 1) c / 256 in cell units (exact), so a brick of B texels spans
+// floor(q1) - floor(q0) = max(B c / 128 - 1, 0) cells at every position: compile-time boxes.
+//
+// Each work-item takes four consecutive texels along x. They share their home cell at 9 of the 12 Worley levels
+// (cells of 4 texels or more), two by two at 64 cells an axis and step one cell each at 128, so every cell's
+// position is read from LDS once for the four, and its y and z differences are squared once: per texel and cell
+// 5 operations instead of 9 and a quarter to a half of a read. One texel per work-item was bound by its
+// 356 16-byte LDS reads: 250 us a volume, now 128-140, of which about 80 are the distances' vector operations.
+constexpr int k128X = 16, k128Y = 8, k128Z = 8, k128T = 4;
+constexpr int k128Span(int l, int b) { return b * low_level_cells(l) / 128 >= 1 ? b * low_level_cells(l) / 128 - 1 : 0; }
+constexpr int k128N(int l, int b) { return k128Span(l, b) + 2 + (l < 4 ? 0 : 1); }
+constexpr int k128Cells(int l) { return k128N(l, k128X) * k128N(l, k128Y) * k128N(l, k128Z); }
+constexpr int k128Off(int l) { return l == 0 ? 0 : k128Off(l - 1) + k128Cells(l - 1); }
+static_assert(k128N(15, 16) == 18 && k128N(15, 8) == 10 && k128N(0, 8) == 2, "128^3 staged box sizes");
+static_assert(k128X / k128T * k128Y * k128Z == 256, "four texels per work-item");
+// Home cell of texel t of a work-item's four, relative to the first's.
+constexpr int k128Shift(int l, int t) { return low_level_cells(l) == 128 ? t : low_level_cells(l) == 64 ? t / 2 : 0; }
+
+// First cell of level l's box on an axis: floor(q(t0)) - pad for a brick starting at texel t0.
+template <int L>
+__device__ __forceinline__ int origin128(int t0) { return ((t0 * low_level_cells(L)) >> 7) - (L < 4 ? 0 : 1); }
+
+template <int L>
+__device__ __forceinline__ void stage128(float4* cells, uint32_t seed, int x0, int y0, int z0) {
+    constexpr int c = low_level_cells(L), nx = k128N(L, k128X), ny = k128N(L, k128Y), off = k128Off(L), n = k128Cells(L);
+    const uint32_t s = low_level_seed(seed, L);
+    const int bx = origin128<L>(x0), by = origin128<L>(y0), bz = origin128<L>(z0);
+    for (int e = ((int)threadIdx.x + 64 * L) & 255; e < n; e += 256) {
+        const int jx = e % nx, jy = (e / nx) % ny, jz = e / (nx * ny);
+        float u0, u1, u2;
+        if constexpr (L < 4) HashGrads{c, s}.point(bx + jx, by + jy, bz + jz, u0, u1, u2);
+        else HashCells{c, s}.point(bx + jx, by + jy, bz + jz, u0, u1, u2);
+        cells[off + e] = make_float4(u0, u1, u2, 0.0f);
     }
+    if constexpr (L + 1 < kLowLevels) stage128<L + 1>(cells, seed, x0, y0, z0);
+}
+
+// worley_at for the four texels: the same arithmetic for each.
+template <int L>
+__device__ __forceinline__ void worley128(const float4* cells, const float (&px)[k128T], float py, float pz, int x0,
+                                          int y0, int z0, float (&out)[k128T]) {
+    constexpr int c = low_level_cells(L), nx = k128N(L, k128X), ny = k128N(L, k128Y), off = k128Off(L);
+    const float qy = py * (float)c, qz = pz * (float)c;
+    const int iy = (int)floorf(qy), iz = (int)floorf(qz), ix = (int)floorf(px[0] * (float)c);
+    const float4* home = cells + off + ((iz - origin128<L>(z0)) * ny + (iy - origin128<L>(y0))) * nx + (ix - origin128<L>(x0));
+    float bx[k128T][3], best[k128T];
+#pragma unroll
+    for (int t = 0; t < k128T; t++) {
+        best[t] = 1e30f;
+#pragma unroll
+        for (int o = 0; o < 3; o++) bx[t][o] = px[t] * (float)c - (float)(ix + k128Shift(L, t) + o - 1);
+    }
+    // a loop: twelve levels unrolled in full would not fit the instruction cache
+#pragma unroll 1
+    for (int oz = -1; oz <= 1; oz++) {
+        const float bz = qz - (float)(iz + oz);
+#pragma unroll
+        for (int oy = -1; oy <= 1; oy++) {
+            const float by = qy - (float)(iy + oy);
+#pragma unroll
+            for (int j = 0; j < 3 + k128Shift(L, k128T - 1); j++) {
+                const float4 u = home[(oz * ny + oy) * nx + j - 1];
+                const float dy = by - u.y, dz = bz - u.z;
+                const float dy2 = dy * dy, dz2 = dz * dz;
+#pragma unroll
+                for (int t = 0; t < k128T; t++) {
+                    const int o = j - k128Shift(L, t);
+                    if (o < 0 || o > 2) continue;
+                    const float dx = bx[t][o] - u.x;
+                    best[t] = __builtin_fminf(((dx * dx) + dy2) + dz2, best[t]);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < k128T; t++) {
+        const float d = sqrt_rn(best[t]);
+        out[t] = 1.0f - (d < 1.0f ? d : 1.0f);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // one level's reads in flight at a time: the levels together would spill
+}
+
+// perlin_at for the four texels, which share their lattice cell at every Perlin level.
+template <int L>
+__device__ __forceinline__ void perlin128(const float4* cells, const float (&px)[k128T], float py, float pz, int x0,
+                                          int y0, int z0, float (&out)[k128T]) {
+    constexpr int c = low_level_cells(L), nx = k128N(L, k128X), ny = k128N(L, k128Y), off = k128Off(L);
+    const float qy = py * (float)c, qz = pz * (float)c;
+    const float fx = floorf(px[0] * (float)c), fy = floorf(qy), fz = floorf(qz);
+    const float ry = qy - fy, rz = qz - fz, uy = fade(ry), uz = fade(rz);
+    const float4* home = cells + off + (((int)fz - origin128<L>(z0)) * ny + ((int)fy - origin128<L>(y0))) * nx +
+                         ((int)fx - origin128<L>(x0));
+    float4 g[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) g[k] = home[((k >> 2) * ny + ((k >> 1) & 1)) * nx + (k & 1)];
+#pragma unroll
+    for (int t = 0; t < k128T; t++) {
+        const float rx = px[t] * (float)c - fx, ux = fade(rx);
+        float n[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float ax = rx - (float)(k & 1), ay = ry - (float)((k >> 1) & 1), az = rz - (float)(k >> 2);
+            n[k] = ((g[k].x * ax) + (g[k].y * ay)) + (g[k].z * az);
+        }
+        const float x00 = lerp_(n[0], n[1], ux), x10 = lerp_(n[2], n[3], ux);
+        const float x01 = lerp_(n[4], n[5], ux), x11 = lerp_(n[6], n[7], ux);
+        out[t] = lerp_(lerp_(x00, x10, uy), lerp_(x01, x11, uy), uz);
+    }
+}
+
+template <int LY>
+__device__ __forceinline__ void layer128(const float4* cells, const float (&px)[k128T], float py, float pz, int x0,
+                                         int y0, int z0, const float (&perlin)[k128T], float (&v)[k128T][4]) {
+    float a[k128T], b[k128T], c[k128T];
+    worley128<4 + 3 * LY>(cells, px, py, pz, x0, y0, z0, a);
+    worley128<5 + 3 * LY>(cells, px, py, pz, x0, y0, z0, b);
+    worley128<6 + 3 * LY>(cells, px, py, pz, x0, y0, z0, c);
+#pragma unroll
+    for (int t = 0; t < k128T; t++) {
+        const float wf = worley_mix(a[t], b[t], c[t]);
+        v[t][LY] = LY == 0 ? perlin_worley_channel(perlin[t], wf) : worley_channel(wf);
+    }
+    if constexpr (LY < 3) layer128<LY + 1>(cells, px, py, pz, x0, y0, z0, perlin, v);
+}
+
+template <int L>
+__device__ __forceinline__ void perlin_fbm128(const float4* cells, const float (&px)[k128T], float py, float pz, int x0,
+                                              int y0, int z0, float w, float (&s)[k128T]) {
+    float p[k128T];
+    perlin128<L>(cells, px, py, pz, x0, y0, z0, p);
+#pragma unroll
+    for (int t = 0; t < k128T; t++) s[t] = s[t] + w * p[t];
+    if constexpr (L < 3) perlin_fbm128<L + 1>(cells, px, py, pz, x0, y0, z0, w * 0.5f, s);
+}
+
+__global__ __launch_bounds__(256, 3) void low_res_128_kernel(GenArgs a) {
+    __shared__ float4 cells[k128Off(kLowLevels)];
+    constexpr int dim = 128, nbx = dim / k128X, nby = dim / k128Y;
+    const int b = (int)blockIdx.x, tid = (int)threadIdx.x;
+    const int x0 = (b % nbx) * k128X, y0 = (b / nbx % nby) * k128Y, z0 = b / (nbx * nby) * k128Z;
+    stage128<0>(cells, a.seed, x0, y0, z0);
+    __syncthreads();
+    const int x = x0 + (tid % (k128X / k128T)) * k128T, y = y0 + tid / (k128X / k128T) % k128Y,
+              z = z0 + tid / (k128X / k128T * k128Y);
+    constexpr float inv = 1.0f / (2 * dim);
+    float px[k128T];
+#pragma unroll
+    for (int t = 0; t < k128T; t++) px[t] = (float)(2 * (x + t) + 1) * inv;
+    const float py = (float)(2 * y + 1) * inv, pz = (float)(2 * z + 1) * inv;
+    float perlin[k128T] = {}, v[k128T][4];
+    perlin_fbm128<0>(cells, px, py, pz, x0, y0, z0, 1.0f, perlin);
+#pragma unroll
+    for (int t = 0; t < k128T; t++) perlin[t] = perlin[t] * (1.0f / 1.875f);
+    layer128<0>(cells, px, py, pz, x0, y0, z0, perlin, v);
+    uint32_t word[k128T];
+#pragma unroll
+    for (int t = 0; t < k128T; t++) word[t] = encode_low_res(a, v[t]);
+    const long sd = dim + a.apron;
+    for (int zs = z; zs < sd; zs += dim)
+        for (int ys = y; ys < sd; ys += dim) {
+            uint32_t* row = reinterpret_cast<uint32_t*>(a.dst) + ((long)zs * sd + ys) * sd + x;
+#pragma unroll
+            for (int t = 0; t < k128T; t++) row[t] = word[t];
+            if (x + dim < sd) row[dim] = word[0];  // the apron repeats texel 0 (x is a multiple of 4)
+        }
 }
 
 __global__ __launch_bounds__(256) void weather_kernel(GenArgs a) {
@@ -719,6 +820,27 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
 }
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + 255) / 256); }
+
+// volume_brick_kernel over every brick, with the LDS its staged levels can need (any brick's boxes are within
+// the bound, so what fits it on the host fits it in the kernel).
+template <bool HI>
+void launch_bricks(const GenArgs& a, hipStream_t s) {
+    // the most cells a layer's levels can take together; a larger level may still be staged in what others leave
+    long cap = 0;
+    for (int l0 = 0; l0 < (HI ? kHiLevels : kLowLevels); l0 += HI || l0 ? 3 : 4) {
+        long layer = 0;
+        for (int l = l0; l < l0 + (HI || l0 ? 3 : 4); l++) {
+            const int c = HI ? hi_level_cells(l) : low_level_cells(l), pad = HI || l >= 4 ? 1 : 0;
+            layer += box_bound(kBrickX, a.dim, c, pad) * box_bound(kBrickY, a.dim, c, pad) * box_bound(kBrickZ, a.dim, c, pad);
+        }
+        cap = std::max(cap, layer);
+    }
+    cap = std::min<long>(cap, kStageCap);
+    const long bricks = (long)((a.dim + kBrickX - 1) / kBrickX) * ((a.dim + kBrickY - 1) / kBrickY) *
+                        ((a.dim + kBrickZ - 1) / kBrickZ);
+    hipLaunchKernelGGL(volume_brick_kernel<HI>, dim3((unsigned)bricks), dim3(256), (size_t)cap * sizeof(float4), s, a,
+                       (int)cap);
+}
 
 }  // namespace
 
@@ -869,8 +991,7 @@ int launch_generate(const mm_noise_params* p, const mm_noise_set* out, void* wor
     if (p->what & MM_GEN_HI_RES) {
         const mm_texture& t = out->hi_res;
         GenArgs a{(uint8_t*)t.data, t.width, t.layout == MM_LAYOUT_APRON ? 1 : 0, t.format, p->seed, 0.f, {1, 1, 1, 1}};
-        const long sd = t.width + a.apron;
-        hipLaunchKernelGGL(hi_res_kernel, dim3(blocks_for(sd * sd * sd)), dim3(256), 0, s, a);
+        launch_bricks<true>(a, s);
     }
     if (p->what & MM_GEN_WEATHER) {
         const mm_texture& t = out->weather;
@@ -884,12 +1005,8 @@ int launch_generate(const mm_noise_params* p, const mm_noise_set* out, void* wor
         GenArgs a{(uint8_t*)t.data, t.width, t.layout == MM_LAYOUT_APRON ? 1 : 0, t.format, p->seed, 0.f, {1, 1, 1, 1}};
         if (t.format == MM_FMT_FP8X4)
             for (int k = 0; k < 4; k++) a.inv_scale[k] = 1.0f / t.scale[k];
-        const long bricks = (long)((t.width + kBrickX - 1) / kBrickX) * ((t.width + kBrickY - 1) / kBrickY) *
-                            ((t.width + kBrickZ - 1) / kBrickZ);
-        if (t.width == 128)
-            hipLaunchKernelGGL(low_res_brick_kernel<true>, dim3((unsigned)bricks), dim3(256), 0, main, a);
-        else
-            hipLaunchKernelGGL(low_res_brick_kernel<false>, dim3((unsigned)bricks), dim3(256), 0, main, a);
+        if (t.width == 128) hipLaunchKernelGGL(low_res_128_kernel, dim3(128 / k128X * (128 / k128Y) * (128 / k128Z)), dim3(256), 0, main, a);
+        else launch_bricks<false>(a, main);
     }
     if (side) {
         const int e = side_join(main, side);
