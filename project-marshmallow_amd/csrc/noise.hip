@@ -42,8 +42,10 @@ __device__ __forceinline__ double sin_poly(double x) {
     return -c;
 }
 
-__global__ void curl_table_kernel(uint8_t* __restrict__ table) {
+// Also resets the min / max cells of the field kernel that follows (mm: 3 x (min, max), see f2ord).
+__global__ void curl_table_kernel(uint8_t* __restrict__ table, uint32_t* __restrict__ mm) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < 6) mm[i] = i & 1 ? 0u : 0xffffffffu;
     if (i >= kLat * kLat * kLat) return;
     const float x = (float)(i % kLat - kLatOff), y = (float)((i / kLat) % kLat - kLatOff),
                 z = (float)(i / (kLat * kLat) - kLatOff);
@@ -121,51 +123,58 @@ __device__ __forceinline__ float ord2f(uint32_t u) {
     return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
 }
 
-// curlNoiseFBM (ImageUtils.cpp:130-169) per texel + block min/max.
-__global__ __launch_bounds__(256) void curl_field_kernel(const uint8_t* __restrict__ tab, int dim,
-                                                         float* __restrict__ field, uint32_t* __restrict__ mm) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    if (i < dim * dim) {
+// curlNoiseFBM (ImageUtils.cpp:130-169) + min/max. A chain of dependent FP64 lerps: latency bounds it, not the
+// arithmetic. A block takes 64 texels and six waves, one per partial derivative (two FBMs, eight Perlin
+// evaluations); the first wave combines them. 128^2: 19-24 us, against 53-60 with a work-item per texel (256
+// waves of 48 Perlin evaluations each on 1024 SIMDs).
+constexpr int kCurlTexels = 64;
+__global__ __launch_bounds__(6 * kCurlTexels) void curl_field_kernel(const uint8_t* __restrict__ tab, int dim,
+                                                                     float* __restrict__ field,
+                                                                     uint32_t* __restrict__ mm) {
+    __shared__ float part[6][kCurlTexels];
+    const int lane = threadIdx.x & 63, d = threadIdx.x >> 6, i = blockIdx.x * kCurlTexels + lane;
+    const bool in = i < dim * dim;
+    if (in) {
         const int row = i / dim, col = i % dim;
         const float px = (float)col / (float)dim, py = (float)row / (float)dim;
         const double eps = 0.0005;
         const float xm = (float)((double)px - eps), xp = (float)((double)px + eps);
         const float ym = (float)((double)py - eps), yp = (float)((double)py + eps);
-        const float f = 3.f;
-        const int o = 4;
-        float dydx = central(fbm_ref(tab, xm, py, 0.5f, f, o), fbm_ref(tab, xp, py, 0.5f, f, o));
-        float dxdy = central(fbm_ref(tab, px, ym, 0.5f, f, o), fbm_ref(tab, px, yp, 0.5f, f, o));
-        float dxdz = central(fbm_ref(tab, px, 0.5f, ym, f, o), fbm_ref(tab, px, 0.5f, yp, f, o));
-        float dzdx = central(fbm_ref(tab, xm, 0.5f, py, f, o), fbm_ref(tab, xp, 0.5f, py, f, o));
-        float dzdy = central(fbm_ref(tab, 0.5f, ym, px, f, o), fbm_ref(tab, 0.5f, yp, px, f, o));
-        float dydz = central(fbm_ref(tab, 0.5f, py, xm, f, o), fbm_ref(tab, 0.5f, py, xp, f, o));
-        float v[3] = {dzdy - dydz, dxdz - dzdx, dydx - dxdy};
+        // the derivatives' two points: 0 dydx, 1 dxdy, 2 dxdz, 3 dzdx, 4 dzdy, 5 dydz
+        float a[3], b[3];
+        switch (d) {
+            case 0: a[0] = xm; b[0] = xp; a[1] = b[1] = py; a[2] = b[2] = 0.5f; break;
+            case 1: a[0] = b[0] = px; a[1] = ym; b[1] = yp; a[2] = b[2] = 0.5f; break;
+            case 2: a[0] = b[0] = px; a[1] = b[1] = 0.5f; a[2] = ym; b[2] = yp; break;
+            case 3: a[0] = xm; b[0] = xp; a[1] = b[1] = 0.5f; a[2] = b[2] = py; break;
+            case 4: a[0] = b[0] = 0.5f; a[1] = ym; b[1] = yp; a[2] = b[2] = px; break;
+            default: a[0] = b[0] = 0.5f; a[1] = b[1] = py; a[2] = xm; b[2] = xp; break;
+        }
+        part[d][lane] = central(fbm_ref(tab, a[0], a[1], a[2], 3.f, 4), fbm_ref(tab, b[0], b[1], b[2], 3.f, 4));
+    }
+    __syncthreads();
+    if (d != 0) return;
+    float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    if (in) {
+        const float v[3] = {part[4][lane] - part[5][lane], part[2][lane] - part[3][lane], part[0][lane] - part[1][lane]};
         for (int k = 0; k < 3; k++) {
             field[3 * i + k] = v[k];
             lo[k] = v[k];
             hi[k] = v[k];
         }
     }
-    // wave reduction, then one atomic per wave and channel
+    // wave reduction, then one atomic per block and channel
     for (int k = 0; k < 3; k++) {
         for (int off = 32; off > 0; off >>= 1) {
             lo[k] = fminf(lo[k], __shfl_xor(lo[k], off));
             hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], off));
         }
     }
-    if ((threadIdx.x & 63) == 0) {
+    if (lane == 0) {
         for (int k = 0; k < 3; k++) {
             atomicMin(&mm[2 * k], f2ord(lo[k]));
             atomicMax(&mm[2 * k + 1], f2ord(hi[k]));
         }
-    }
-}
-
-__global__ void curl_minmax_init_kernel(uint32_t* mm) {
-    if (threadIdx.x < 3) {
-        mm[2 * threadIdx.x] = 0xffffffffu;
-        mm[2 * threadIdx.x + 1] = 0u;
     }
 }
 
@@ -980,9 +989,9 @@ int launch_generate(const mm_noise_params* p, const mm_noise_set* out, void* wor
         uint32_t* mmx = (uint32_t*)(ws + 20480);
         float* field = (float*)(ws + 20480 + 256);
         const int dim = t.width;
-        hipLaunchKernelGGL(curl_table_kernel, dim3(blocks_for(kLat * kLat * kLat)), dim3(256), 0, s, table);
-        hipLaunchKernelGGL(curl_minmax_init_kernel, dim3(1), dim3(64), 0, s, mmx);
-        hipLaunchKernelGGL(curl_field_kernel, dim3(blocks_for((long)dim * dim)), dim3(256), 0, s, table, dim, field, mmx);
+        hipLaunchKernelGGL(curl_table_kernel, dim3(blocks_for(kLat * kLat * kLat)), dim3(256), 0, s, table, mmx);
+        hipLaunchKernelGGL(curl_field_kernel, dim3((unsigned)((dim * dim + kCurlTexels - 1) / kCurlTexels)),
+                           dim3(6 * kCurlTexels), 0, s, table, dim, field, mmx);
         const int apron = t.layout == MM_LAYOUT_APRON ? 1 : 0;
         const long n = (long)(dim + apron) * (dim + apron);
         hipLaunchKernelGGL(curl_store_kernel, dim3(blocks_for(n)), dim3(256), 0, s, field, mmx, dim, apron, t.format,
