@@ -258,6 +258,13 @@ struct LdsCells {
     }
 };
 
+// A lower bound of fl((b - u)^2) over u in [0, 1], with the same roundings (each is monotone): no cell of a row
+// whose bounds in y and z sum to `best` or more can lower it, so the row is skipped and the minimum is the same.
+__device__ __forceinline__ float near_sq(float b) {
+    const float d = __builtin_fmaxf(__builtin_fmaxf(b - 1.0f, -b), 0.0f);
+    return d * d;
+}
+
 // Inverted F1 cellular noise on a periodic grid of `cells`^3 cells.
 template <class Cells>
 __device__ __forceinline__ float worley_at(float px, float py, float pz, int cells, const Cells& src) {
@@ -611,12 +618,21 @@ __global__ __launch_bounds__(256) void volume_brick_kernel(GenArgs a, int cap) {
 // (cells of 4 texels or more), two by two at 64 cells an axis and step one cell each at 128, so every cell's
 // position is read from LDS once for the four, and its y and z differences are squared once: per texel and cell
 // 5 operations instead of 9 and a quarter to a half of a read. One texel per work-item was bound by its
-// 356 16-byte LDS reads: 250 us a volume, now 128-140, of which about 80 are the distances' vector operations.
+// 356 16-byte LDS reads: 250 us a volume, now 114-127, of which about 70 are the distances' vector operations.
+// 36 KB of LDS and at most 128 registers, so that four blocks share a CU: 2 x 1024 blocks fill the chip twice
+// (three a CU, all levels staged at once: 128-140 us, and the small grids of the other maps waited for slots).
 constexpr int k128X = 16, k128Y = 8, k128Z = 8, k128T = 4;
 constexpr int k128Span(int l, int b) { return b * low_level_cells(l) / 128 >= 1 ? b * low_level_cells(l) / 128 - 1 : 0; }
 constexpr int k128N(int l, int b) { return k128Span(l, b) + 2 + (l < 4 ? 0 : 1); }
 constexpr int k128Cells(int l) { return k128N(l, k128X) * k128N(l, k128Y) * k128N(l, k128Z); }
-constexpr int k128Off(int l) { return l == 0 ? 0 : k128Off(l - 1) + k128Cells(l - 1); }
+// Levels are staged layer by layer (Perlin 0..3, then three Worley levels at a time) into the same cells.
+constexpr bool k128First(int l) { return l == 0 || (l >= 4 && (l - 4) % 3 == 0); }
+constexpr int k128Off(int l) { return k128First(l) ? 0 : k128Off(l - 1) + k128Cells(l - 1); }
+constexpr int k128LdsCells() {
+    int n = 0;
+    for (int l = 0; l < kLowLevels; l++) n = k128Off(l) + k128Cells(l) > n ? k128Off(l) + k128Cells(l) : n;
+    return n;
+}
 static_assert(k128N(15, 16) == 18 && k128N(15, 8) == 10 && k128N(0, 8) == 2, "128^3 staged box sizes");
 static_assert(k128X / k128T * k128Y * k128Z == 256, "four texels per work-item");
 // Home cell of texel t of a work-item's four, relative to the first's.
@@ -638,7 +654,7 @@ __device__ __forceinline__ void stage128(float4* cells, uint32_t seed, int x0, i
         else HashCells{c, s}.point(bx + jx, by + jy, bz + jz, u0, u1, u2);
         cells[off + e] = make_float4(u0, u1, u2, 0.0f);
     }
-    if constexpr (L + 1 < kLowLevels) stage128<L + 1>(cells, seed, x0, y0, z0);
+    if constexpr (L + 1 < kLowLevels && !k128First(L + 1)) stage128<L + 1>(cells, seed, x0, y0, z0);
 }
 
 // worley_at for the four texels: the same arithmetic for each.
@@ -656,17 +672,26 @@ __device__ __forceinline__ void worley128(const float4* cells, const float (&px)
 #pragma unroll
         for (int o = 0; o < 3; o++) bx[t][o] = px[t] * (float)c - (float)(ix + k128Shift(L, t) + o - 1);
     }
+    float by[3], ly[3];
+#pragma unroll
+    for (int o = 0; o < 3; o++) {
+        by[o] = qy - (float)(iy + o - 1);
+        ly[o] = near_sq(by[o]);
+    }
+    float far = 1e30f;
     // a loop: twelve levels unrolled in full would not fit the instruction cache
 #pragma unroll 1
-    for (int oz = -1; oz <= 1; oz++) {
-        const float bz = qz - (float)(iz + oz);
+    for (int k = 0; k < 3; k++) {  // slabs 0, -1, +1
+        const int oz = k == 0 ? 0 : 2 * k - 3;
+        const float bz = qz - (float)(iz + oz), lz = near_sq(bz);
 #pragma unroll
-        for (int oy = -1; oy <= 1; oy++) {
-            const float by = qy - (float)(iy + oy);
+        for (int r = 0; r < 3; r++) {  // rows 0, -1, +1
+            const int o1 = r == 0 ? 1 : 2 * r - 2;
+            if (!(ly[o1] + lz < far)) continue;
 #pragma unroll
             for (int j = 0; j < 3 + k128Shift(L, k128T - 1); j++) {
-                const float4 u = home[(oz * ny + oy) * nx + j - 1];
-                const float dy = by - u.y, dz = bz - u.z;
+                const float4 u = home[(oz * ny + o1 - 1) * nx + j - 1];
+                const float dy = by[o1] - u.y, dz = bz - u.z;
                 const float dy2 = dy * dy, dz2 = dz * dz;
 #pragma unroll
                 for (int t = 0; t < k128T; t++) {
@@ -676,6 +701,7 @@ __device__ __forceinline__ void worley128(const float4* cells, const float (&px)
                     best[t] = __builtin_fminf(((dx * dx) + dy2) + dz2, best[t]);
                 }
             }
+            far = __builtin_fmaxf(__builtin_fmaxf(best[0], best[1]), __builtin_fmaxf(best[2], best[3]));
         }
     }
 #pragma unroll
@@ -715,9 +741,12 @@ __device__ __forceinline__ void perlin128(const float4* cells, const float (&px)
 }
 
 template <int LY>
-__device__ __forceinline__ void layer128(const float4* cells, const float (&px)[k128T], float py, float pz, int x0,
+__device__ __forceinline__ void layer128(float4* cells, uint32_t seed, const float (&px)[k128T], float py, float pz, int x0,
                                          int y0, int z0, const float (&perlin)[k128T], float (&v)[k128T][4]) {
     float a[k128T], b[k128T], c[k128T];
+    __syncthreads();  // the last layer's cells are no longer read
+    stage128<4 + 3 * LY>(cells, seed, x0, y0, z0);
+    __syncthreads();
     worley128<4 + 3 * LY>(cells, px, py, pz, x0, y0, z0, a);
     worley128<5 + 3 * LY>(cells, px, py, pz, x0, y0, z0, b);
     worley128<6 + 3 * LY>(cells, px, py, pz, x0, y0, z0, c);
@@ -726,7 +755,7 @@ __device__ __forceinline__ void layer128(const float4* cells, const float (&px)[
         const float wf = worley_mix(a[t], b[t], c[t]);
         v[t][LY] = LY == 0 ? perlin_worley_channel(perlin[t], wf) : worley_channel(wf);
     }
-    if constexpr (LY < 3) layer128<LY + 1>(cells, px, py, pz, x0, y0, z0, perlin, v);
+    if constexpr (LY < 3) layer128<LY + 1>(cells, seed, px, py, pz, x0, y0, z0, perlin, v);
 }
 
 template <int L>
@@ -736,11 +765,12 @@ __device__ __forceinline__ void perlin_fbm128(const float4* cells, const float (
     perlin128<L>(cells, px, py, pz, x0, y0, z0, p);
 #pragma unroll
     for (int t = 0; t < k128T; t++) s[t] = s[t] + w * p[t];
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (L < 3) perlin_fbm128<L + 1>(cells, px, py, pz, x0, y0, z0, w * 0.5f, s);
 }
 
-__global__ __launch_bounds__(256, 3) void low_res_128_kernel(GenArgs a) {
-    __shared__ float4 cells[k128Off(kLowLevels)];
+__global__ __launch_bounds__(256, 4) void low_res_128_kernel(GenArgs a) {
+    __shared__ float4 cells[k128LdsCells()];
     constexpr int dim = 128, nbx = dim / k128X, nby = dim / k128Y;
     const int b = (int)blockIdx.x, tid = (int)threadIdx.x;
     const int x0 = (b % nbx) * k128X, y0 = (b / nbx % nby) * k128Y, z0 = b / (nbx * nby) * k128Z;
@@ -756,8 +786,11 @@ __global__ __launch_bounds__(256, 3) void low_res_128_kernel(GenArgs a) {
     float perlin[k128T] = {}, v[k128T][4];
     perlin_fbm128<0>(cells, px, py, pz, x0, y0, z0, 1.0f, perlin);
 #pragma unroll
-    for (int t = 0; t < k128T; t++) perlin[t] = perlin[t] * (1.0f / 1.875f);
-    layer128<0>(cells, px, py, pz, x0, y0, z0, perlin, v);
+    for (int t = 0; t < k128T; t++) {
+        perlin[t] = perlin[t] * (1.0f / 1.875f);
+        asm volatile("" : "+v"(perlin[t]));  // computed here: sunk to its use, it would hold 96 registers of gradients
+    }
+    layer128<0>(cells, a.seed, px, py, pz, x0, y0, z0, perlin, v);
     uint32_t word[k128T];
 #pragma unroll
     for (int t = 0; t < k128T; t++) word[t] = encode_low_res(a, v[t]);
