@@ -277,18 +277,21 @@ def noise_block(ns, noise_ms):
 
 def march_kernel_name(args):
     """The kernel a full-frame plain march launches: lock-step, cone-batched (1 lane per ray: the
-    default of a scheduled march) or ray-parallel (2 lanes per ray: the unscheduled default)."""
+    default of a scheduled 1080p march) or ray-parallel (2 lanes per ray: its unscheduled default)."""
     if args.no_batch:
         return "march_kernel"
-    lanes = args.lanes_per_ray or (2 if args.no_schedule else 1)
-    return "march_batched_kernel" if lanes == 1 else "march_rp_kernel"
+    return "march_batched_kernel" if lanes_and_tiles(args)[0] == 1 else "march_rp_kernel"
 
 
 def lanes_and_tiles(args):
     """(lanes per ray, tile width) the launch runs with (the library's defaults when 0)."""
     if args.no_batch:
         return 1, args.tile_width or 8
-    lanes = args.lanes_per_ray or (2 if args.no_schedule else 1)
+    rays = getattr(args, "width", 1920) * getattr(args, "height", 1080)
+    if args.no_schedule:
+        lanes = args.lanes_per_ray or (8 if rays <= 400_000 else 2)
+    else:
+        lanes = args.lanes_per_ray or (8 if rays <= 200_000 else 4 if rays <= 480_000 else 2 if rays <= 1 << 20 else 1)
     if lanes > 1:
         return lanes, 8
     return 1, args.tile_width or (8 if args.no_schedule else 16)

@@ -216,9 +216,11 @@ typedef struct mm_march_params {
     int32_t tile_width;         /* pixels per wave tile row: 8 (8x8, default when 0), 16 (16x4), 32 (32x2);
                                    the image does not depend on it */
     int32_t lanes_per_ray;      /* 1, 2, 4 or 8 lanes march one ray, sampling the next trips ahead
-                                   and committing them in order (0 = default: 8 for one phase, else
-                                   2); plain cones only (other modes use 1); the image does not
-                                   depend on it */
+                                   and committing them in order (0 = default, by the rays marched:
+                                   8 for a phase of up to 2^19 rays and a frame of up to 400 000, else
+                                   2; through a schedule 8, 4, 2 and 1 from the smallest frames to
+                                   those over 2^20 rays); plain cones only (the surrogate-lit march
+                                   takes at most 2, other modes 1); the image does not depend on it */
     int32_t _reserved[6];
 } mm_march_params;
 
@@ -292,7 +294,8 @@ int mm_march_clouds_state(const mm_camera_ubo* camera, const mm_sun_ubo* sun, co
  * ignores it.
  * mm_march_schedule_create allocates device buffers for up to max_tiles tiles (a full 1920x1080
  * frame has 32400 at the scheduled default of one lane per ray in 16 x 4 tiles, 64800 at two lanes
- * per ray); launches with more tiles return MM_E_SIZE, and
+ * per ray). The default lanes per ray of a smaller frame are lowered until its tiles fit; launches
+ * with more tiles return MM_E_SIZE, and
  * a schedule is used on the device that created it. Launches that share a schedule must be ordered
  * (one stream): the order buffer is rewritten by each. */
 typedef struct mm_march_schedule mm_march_schedule;

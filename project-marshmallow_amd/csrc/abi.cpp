@@ -275,10 +275,18 @@ struct CollectArgs {
 
 // Validates one dispatch and derives its per-dispatch constants and texture views. `empty` is set
 // when the phase selects no pixel of the image (nothing to launch).
-// Default lanes per ray (see ray_parallel_tiles), measured on the 1080p scenario frame: every pixel
-// 1 / 2 / 4 / 8 lanes 1.85 / 1.73 / 2.07 / 2.91 ms; one 1/16 phase 0.93 / 0.56 / 0.40 / 0.33 ms.
-constexpr int kDefaultFrameLanesPerRay = 2;
-constexpr int kDefaultPhaseLanesPerRay = 8;
+// Default lanes per ray, by the number of rays marched. A launch of few rays lasts as long as its longest
+// ray, whose chain of samples more lanes shorten; with many rays the chip is full and the trips sampled
+// ahead in vain cost more. Both scenes (scenario / reference preset), us at 1, 2, 4, 8 lanes:
+//   unscheduled  65 536 rays  808 418 225 142 / 505 282 166 114;  324 000: 2, 4, 8: 530 358 315 / 363 354 337;
+//     409 920: 569 379 397 / 415 354 415;  518 400: 921 632 547 489 / 676 464 492 517;
+//     921 600: 1256 752 872 896 / 977 727 758 966
+//   with a schedule (longest tiles first)  65 536: 752 433 241 153 / 529 292 164 112;
+//     230 400: 839 491 269 247 / 573 335 209 247;  518 400: 785 459 420 473 / 622 384 394 506;
+//     921 600: 807 641 712 820 / 681 616 653 872;  1 440 000: 915 964 1087 1268 / 853 913 985 1341
+//   one phase  518 400: 826 600 549 459 / 613 401 475 467;  921 600: 1137 684 855 841 / 875 617 727 874
+constexpr long long kFrameRays8 = 400000, kPhaseRays8 = 1 << 19;
+constexpr long long kScheduledRays8 = 200000, kScheduledRays4 = 480000, kScheduledRays2 = 1 << 20;
 // A views launch has many more waves (64 views of 256x256 to 1920x1080: 33.6 M pixels, 1 / 2 / 4
 // lanes 20.4 / 21.7 / 29.1 ms): latency is hidden already and one lane per ray wastes no samples.
 constexpr int kDefaultViewsLanesPerRay = 1;
@@ -471,15 +479,35 @@ static int build_march(const mm_camera_ubo* camera, const mm_sun_ubo* sun, const
     return MM_OK;
 }
 
-// Lanes per ray of a plain march (params.lanes_per_ray; 0 = the default: 8 for a single 1/16 phase,
-// where there are few waves and each lasts as long as its longest ray, else 2); 1 for the other cone
-// modes and the lock-step kernel. The image does not depend on it.
+// Per-tile cost history of one launch shape (mm_march_clouds_scheduled).
+struct mm_march_schedule {
+    int capacity = 0;              // tiles the buffers hold
+    unsigned* d_sched = nullptr;   // device record: order state, then each physical tile's cost in the last launch
+    int* d_order = nullptr;        // device: the order built for the current launch
+    bool history = false;          // d_sched holds the costs of a launch of shape `key`
+    int key[6] = {0, 0, 0, 0, 0, 0};
+    int device = 0;
+};
+
+// Lanes per ray of a march (params.lanes_per_ray; 0 = by the rays, see kFrameRays8); 1 for the other cone
+// modes and the lock-step kernel. A schedule takes no more lanes than its record holds the tiles of (the
+// one-lane tiles are the fewest). The image does not depend on it.
 static int lanes_for(const mm::MarchConsts& c, const mm_march_params* params, int32_t phase,
-                     bool scheduled = false) {
+                     const mm_march_schedule* sched = nullptr) {
     int lpr = params ? params->lanes_per_ray : 0;
     const bool one_phase = phase >= 0 || phase == MM_PHASE_FROM_UBO;
-    if (lpr == 0)
-        lpr = one_phase ? kDefaultPhaseLanesPerRay : (scheduled ? 1 : kDefaultFrameLanesPerRay);
+    if (lpr == 0) {
+        const long long rays = (long long)c.gridW * c.gridH;
+        if (one_phase) {
+            lpr = sched || rays <= kPhaseRays8 ? 8 : 2;
+        } else if (!sched) {
+            lpr = rays <= kFrameRays8 ? 8 : 2;
+        } else {
+            lpr = rays <= kScheduledRays8 ? 8 : rays <= kScheduledRays4 ? 4 : rays <= kScheduledRays2 ? 2 : 1;
+            while (lpr > 1 && ((c.gridW + 7) / 8) * (long long)((c.gridH + 8 / lpr - 1) / (8 / lpr)) > sched->capacity)
+                lpr /= 2;
+        }
+    }
     if (c.flags & MM_MARCH_NO_BATCH) return 1;
     // the surrogate-lit march runs with one or two lanes per ray; the sample recorder with one
     if (c.coneMode == MM_CONE_SURROGATE) return lpr >= 2 ? 2 : 1;
@@ -500,16 +528,6 @@ static void set_lanes(mm::MarchConsts& c, int lpr) {
     }
     horizon_first_rows(c);
 }
-
-// Per-tile cost history of one launch shape (mm_march_clouds_scheduled).
-struct mm_march_schedule {
-    int capacity = 0;              // tiles the buffers hold
-    unsigned* d_sched = nullptr;   // device record: order state, then each physical tile's cost in the last launch
-    int* d_order = nullptr;        // device: the order built for the current launch
-    bool history = false;          // d_sched holds the costs of a launch of shape `key`
-    int key[6] = {0, 0, 0, 0, 0, 0};
-    int device = 0;
-};
 
 int mm_march_schedule_create(int32_t max_tiles, mm_march_schedule** schedule) {
     if (!schedule) return MM_E_NULL;
@@ -598,10 +616,10 @@ static int march_impl(const mm_camera_ubo* camera, const mm_sun_ubo* sun, const 
         c.flags |= MM_MARCH_NO_BATCH;
         c.stateOut = state;
     }
-    const int lanes = lanes_for(c, params, phase, sched != nullptr);
+    const int lanes = lanes_for(c, params, phase, sched);
     if (sched && lanes == 1 && (!params || params->tile_width == 0) && phase == MM_PHASE_ALL) {
-        // scheduled full frames default to 16 x 4 tiles (with longest-first order the measured best
-        // shape is one lane per ray in 16-wide tiles)
+        // scheduled full frames of one lane per ray default to 16 x 4 tiles (with longest-first order the
+        // measured best one-lane shape)
         c.tileShift = 4;
         c.tilesX = (c.gridW + 15) >> 4;
         c.tilesY = (c.gridH + 3) / 4;
