@@ -11,8 +11,10 @@
 //                       radial-blur value).
 // The taps of neighbouring pixels overlap, so after the first touch they come from L2. The algorithmic
 // traffic is 16 B read + 4 B written (alpha plane), 4 B read + 4 B written (god rays) and 16 + 4 B
-// read + 4 (or 20) B written (radial blur + tonemap) per pixel; the two tap kernels issue more VALU
-// work per pixel (9 and 11 bilinear taps, exact division) than that traffic takes at HBM rate.
+// read + 4 (or 20) B written (radial blur + tonemap) per pixel. The tap kernels are bound by vector operations
+// and by the caches' lanes: waves whose taps are all inside the image take a tap without clamps and with one
+// 8-byte load a row, and the tonemap of ordinary numbers takes unscaled divisions and no special cases
+// (1080p with the HDR output: god rays 29 us -> 22, blur + tonemap 51 -> 38, the chain 78 -> 62).
 // Arithmetic follows the shaders' evaluation order with IEEE division/sqrt and no contraction; the
 // sampler and the other choices GLSL leaves open are the scalar restatement's, so the result is the
 // same bit for bit.
@@ -26,53 +28,128 @@ namespace {
 
 __device__ __forceinline__ float clampf(float x, float lo, float hi) { return fminf(fmaxf(x, lo), hi); }
 
-// LINEAR / CLAMP_TO_EDGE axis: x = u n - 0.5 rounded to 1/2^bits, i0 = floor(x) and i0 + 1 clamped.
-__device__ __forceinline__ void axis_clamp(float u, int n, int bits, int& i0, int& i1, float& f) {
+// LINEAR / CLAMP_TO_EDGE axis: x = u n - 0.5 rounded to 1/2^bits; i = floor(x) saturated to 32 bits (0 for NaN,
+// whose weight f is NaN), texels i and i + 1, clamped.
+__device__ __forceinline__ void axis(float u, int n, int bits, int& i0, int& i1, float& f) {
     float x = u * (float)n - 0.5f;
     // division by 2^bits is the exact multiplication by 2^-bits (one rounding either way)
     const float s = (float)(1 << bits), inv = __int_as_float((127 - bits) << 23);
     x = floorf(x * s + 0.5f) * inv;
     const float fl = floorf(x);
     f = x - fl;
-    const int i = (int)clampf(fl, -1.0f, (float)n);
+    int i;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(fl));
     i0 = min(max(i, 0), n - 1);
-    i1 = min(max(i + 1, 0), n - 1);
+    i1 = min(max(i, -1), n - 2) + 1;
 }
+
+// Taps of which every texel exists, weights of 1/256 (about 70 issue cycles against 190 for tap_edge): no clamps,
+// one 8-byte load a row. u (256 n) - 128 is 256 times u n - 0.5 with the same roundings, and k = floor(that + 0.5)
+// holds the texel (k >> 8) and 256 times its weight (k & 255); v_cvt_rpi_i32_f32 is the exact floor(v + 0.5),
+// which differs from adding in float only at 0.5 - 2^-25, no difference from 128.
+struct Map {
+    float w256, h256;  // in vector registers: a float instruction with a scalar operand issues at half the rate
+    float right, bottom;
+    uint32_t rowBytes;
+    bool use;  // offsets into the image fit 32 bits, rows and bytes a row 24, 256 n is exact
+};
+__device__ __forceinline__ Map make_map(const mm::PostConsts& c) {
+    Map m;
+    m.w256 = 256.0f * (float)c.width;
+    m.h256 = 256.0f * (float)c.height;
+    asm("" : "+v"(m.w256), "+v"(m.h256));
+    m.right = 256.0f * (float)(c.width - 1) - 1.0f;
+    m.bottom = 256.0f * (float)(c.height - 1) - 1.0f;
+    m.rowBytes = (uint32_t)c.pitch * 4u;
+    m.use = c.bits == 8 && c.width <= 16384 && c.height <= 16384 && c.pitch < (1 << 20) &&
+            (uint64_t)c.pitch * (uint32_t)c.height < (1u << 28);
+    return m;
+}
+struct At {
+    float x, y;  // 256 times the texel coordinates
+};
+__device__ __forceinline__ At locate(const Map& m, float u, float v) { return At{u * m.w256 - 128.0f, v * m.h256 - 128.0f}; }
+// k <= 256 (n - 1) - 1, so k >> 8 <= n - 2; false for NaN.
+__device__ __forceinline__ bool inside(const Map& m, const At& a) {
+    return a.x >= 0.0f && a.y >= 0.0f && a.x <= m.right && a.y <= m.bottom;
+}
+// RN(n / d) from y = RN(1 / d), as div_rn_normal.
+__device__ __forceinline__ float div_by(float n, float d, float y) {
+    float q = n * y;
+    q = __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+}
+__device__ __forceinline__ bool all_lanes(bool b) { return __builtin_amdgcn_ballot_w64(!b) == 0; }
 
 __device__ __forceinline__ float lerp_r(float a, float b, float t) { return a + t * (b - a); }
 
-// Bilinear tap of one float channel: texel (x, y) at byte offset ((y * pitch + x) * step + ch) * 4.
-template <int STEP>
-__device__ __forceinline__ float tap(const float* __restrict__ img, int ch, const mm::PostConsts& c, float u, float v) {
+// Bilinear tap of a plane of floats.
+__device__ __forceinline__ float tap_edge(const float* __restrict__ img, const mm::PostConsts& c, float u, float v) {
     int x0, x1, y0, y1;
     float fx, fy;
-    axis_clamp(u, c.width, c.bits, x0, x1, fx);
-    axis_clamp(v, c.height, c.bits, y0, y1, fy);
+    axis(u, c.width, c.bits, x0, x1, fx);
+    axis(v, c.height, c.bits, y0, y1, fy);
     const uint32_t r0 = (uint32_t)y0 * (uint32_t)c.pitch, r1 = (uint32_t)y1 * (uint32_t)c.pitch;
-    const float t00 = img[(r0 + (uint32_t)x0) * STEP + ch], t01 = img[(r0 + (uint32_t)x1) * STEP + ch];
-    const float t10 = img[(r1 + (uint32_t)x0) * STEP + ch], t11 = img[(r1 + (uint32_t)x1) * STEP + ch];
+    const float t00 = img[r0 + (uint32_t)x0], t01 = img[r0 + (uint32_t)x1];
+    const float t10 = img[r1 + (uint32_t)x0], t11 = img[r1 + (uint32_t)x1];
     return lerp_r(lerp_r(t00, t01, fx), lerp_r(t10, t11, fx), fy);
+}
+__device__ __forceinline__ void texel(const At& a, int& kx, int& ky, float& fx, float& fy) {
+    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(kx) : "v"(a.x));
+    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(ky) : "v"(a.y));
+    fx = (float)(kx & 255) * (1.0f / 256.0f);
+    fy = (float)(ky & 255) * (1.0f / 256.0f);
+}
+__device__ __forceinline__ float tap_inside(const float* __restrict__ img, const Map& m, const At& a) {
+    struct __attribute__((packed, aligned(4))) Pair {
+        float l, r;
+    };
+    int kx, ky;
+    float fx, fy;
+    texel(a, kx, ky, fx, fy);
+    const uint32_t off = __umul24((uint32_t)ky >> 8, m.rowBytes) + (((uint32_t)kx >> 6) & ~3u);
+    const Pair p = *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(img) + off);
+    const Pair q = *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(img) + m.rowBytes + off);
+    return lerp_r(lerp_r(p.l, p.r, fx), lerp_r(q.l, q.r, fx), fy);
 }
 
 // The RGB of one bilinear tap of the RGBA image (one 16-byte load per texel).
-__device__ __forceinline__ void tap_rgb(const float4* __restrict__ img, const mm::PostConsts& c, float u, float v,
-                                        float rgb[3]) {
-    int x0, x1, y0, y1;
-    float fx, fy;
-    axis_clamp(u, c.width, c.bits, x0, x1, fx);
-    axis_clamp(v, c.height, c.bits, y0, y1, fy);
-    const uint32_t r0 = (uint32_t)y0 * (uint32_t)c.pitch, r1 = (uint32_t)y1 * (uint32_t)c.pitch;
-    const float4 t00 = img[r0 + (uint32_t)x0], t01 = img[r0 + (uint32_t)x1];
-    const float4 t10 = img[r1 + (uint32_t)x0], t11 = img[r1 + (uint32_t)x1];
+__device__ __forceinline__ void lerp_rgb(const float4& t00, const float4& t01, const float4& t10, const float4& t11,
+                                         float fx, float fy, float rgb[3]) {
     rgb[0] = lerp_r(lerp_r(t00.x, t01.x, fx), lerp_r(t10.x, t11.x, fx), fy);
     rgb[1] = lerp_r(lerp_r(t00.y, t01.y, fx), lerp_r(t10.y, t11.y, fx), fy);
     rgb[2] = lerp_r(lerp_r(t00.z, t01.z, fx), lerp_r(t10.z, t11.z, fx), fy);
 }
+__device__ __forceinline__ void tap_rgb(const float4* __restrict__ img, const mm::PostConsts& c, const Map& m, float u,
+                                        float v, float rgb[3]) {
+    float fx, fy;
+    const At a = locate(m, u, v);
+    if (m.use && all_lanes(inside(m, a))) {
+        int kx, ky;
+        texel(a, kx, ky, fx, fy);
+        const uint32_t off = __umul24((uint32_t)ky >> 8, m.rowBytes * 4u) + (((uint32_t)kx >> 4) & ~15u);
+        const float4* p = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(img) + off);
+        const float4* q = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(img + c.pitch) + off);
+        lerp_rgb(p[0], p[1], q[0], q[1], fx, fy, rgb);
+        return;
+    }
+    int x0, x1, y0, y1;
+    axis(u, c.width, c.bits, x0, x1, fx);
+    axis(v, c.height, c.bits, y0, y1, fy);
+    const uint32_t r0 = (uint32_t)y0 * (uint32_t)c.pitch, r1 = (uint32_t)y1 * (uint32_t)c.pitch;
+    lerp_rgb(img[r0 + (uint32_t)x0], img[r0 + (uint32_t)x1], img[r1 + (uint32_t)x0], img[r1 + (uint32_t)x1], fx, fy, rgb);
+}
 
 // Uncharted-2 curve (tonemap.frag:11-14) with the shader's constant products folded in float.
+template <bool NORMAL>
+__device__ __forceinline__ float div_rn(float n, float d) {
+    return NORMAL ? div_rn_normal(n, d) : __fdiv_rn(n, d);
+}
+// NORMAL: x in [0, 1e9], so the quotient is in [0.06, 1].
+template <bool NORMAL>
 __device__ __forceinline__ float uc2(float x) {
     const float A = 0.15f, k05 = 0.1f * 0.5f, k004 = 0.2f * 0.02f, k06 = 0.2f * 0.3f, k0067 = 0.02f / 0.3f;
-    return __fdiv_rn(x * (A * x + k05) + k004, x * (A * x + 0.5f) + k06) - k0067;
+    return div_rn<NORMAL>(x * (A * x + k05) + k004, x * (A * x + 0.5f) + k06) - k0067;
 }
 
 // pow(x, y) = exp2(y log2 x), both written out as float operations (the scalar restatement
@@ -81,13 +158,16 @@ __device__ __forceinline__ float uc2(float x) {
 // 2^f = sqrt(2) 2^(f - 1/2) by the exponential series in g = (f - 1/2) ln 2 to g^7, scaled by 2^n
 // exactly. exp2 within 3 ulp, log2 within 1e-6 absolute; pow within 1e-6 relative over the
 // tonemap's inputs (the float rounding of y log2 x dominates); the result is quantised to 8 bits.
+template <bool NORMAL>  // x a positive normal number
 __device__ __forceinline__ float log2_series(float x) {
-    if (!(x > 0.0f)) return x == 0.0f ? -INFINITY : __int_as_float(0x7fc00000);
-    if (x == INFINITY) return INFINITY;
     int e = 0;
-    if (x < 1.17549435e-38f) {  // subnormal: scale into the normal range
-        x = x * 16777216.0f;
-        e = -24;
+    if constexpr (!NORMAL) {
+        if (!(x > 0.0f)) return x == 0.0f ? -INFINITY : __int_as_float(0x7fc00000);
+        if (x == INFINITY) return INFINITY;
+        if (x < 1.17549435e-38f) {  // subnormal: scale into the normal range
+            x = x * 16777216.0f;
+            e = -24;
+        }
     }
     uint32_t b = __float_as_uint(x);
     e += (int)((b >> 23) & 255u) - 127;
@@ -96,7 +176,7 @@ __device__ __forceinline__ float log2_series(float x) {
         m = m * 0.5f;
         e = e + 1;
     }
-    const float s = __fdiv_rn(m - 1.0f, m + 1.0f);
+    const float s = div_rn_normal(m - 1.0f, m + 1.0f);  // 0 or at least 2^-24 by at most 2.5
     const float s2 = s * s;
     float p = 0.320598898f;
     p = p * s2 + 0.412198583f;
@@ -106,10 +186,13 @@ __device__ __forceinline__ float log2_series(float x) {
     return (float)e + s * p;
 }
 
+template <bool NORMAL>  // |t| < 126
 __device__ __forceinline__ float exp2_series(float t) {
-    if (t != t) return t;
-    if (t >= 128.0f) return INFINITY;
-    if (t < -150.0f) return 0.0f;
+    if constexpr (!NORMAL) {
+        if (t != t) return t;
+        if (t >= 128.0f) return INFINITY;
+        if (t < -150.0f) return 0.0f;
+    }
     const float n = floorf(t);
     const float g = ((t - n) - 0.5f) * 0.693147181f;
     float p = 1.98412698e-4f;
@@ -133,14 +216,14 @@ __device__ __forceinline__ bool xcd_tile(const mm::PostConsts& c, int& x, int& y
     const int per = (tiles + 7) >> 3;
     const int t = (int)(blockIdx.x & 7u) * per + (int)(blockIdx.x >> 3);
     if (t >= tiles) return false;
-    x = (t % gx) * 16 + (threadIdx.x & 15);
-    y = (t / gx) * 16 + (threadIdx.x >> 4);
+    const int row = c.tileMagic ? (int)__umulhi((uint32_t)t, c.tileMagic) : t / gx;  // scalar multiply
+    x = (t - row * gx) * 16 + (threadIdx.x & 15);
+    y = row * 16 + (threadIdx.x >> 4);
     return true;
 }
 
 __device__ __forceinline__ uint32_t unorm8(float v) {
-    if (!(v == v)) return 0u;
-    return (uint32_t)floorf(clampf(v, 0.0f, 1.0f) * 255.0f + 0.5f);
+    return (uint32_t)(clampf(v, 0.0f, 1.0f) * 255.0f + 0.5f);  // NaN: fmaxf takes 0
 }
 
 // The image's alpha as a plane of its own: the god-ray taps then read 4-byte texels (32 per
@@ -159,34 +242,56 @@ __global__ __launch_bounds__(256) void god_ray_kernel(const mm::PostConsts c, co
     if (!xcd_tile(c, x, y) || x >= c.width || y >= c.height) return;
     float a = 1.0f;  // sun below the horizon: the pass writes alpha 1 (god-ray.frag:55-57)
     if (!c.below) {
-        const float u = __fdiv_rn((float)x + 0.5f, (float)c.width), v = __fdiv_rn((float)y + 0.5f, (float)c.height);
+        const Map m = make_map(c);
+        const float u = div_by((float)x + 0.5f, (float)c.width, c.rw), v = div_by((float)y + 0.5f, (float)c.height, c.rh);
         float cx = u * 2.0f - 1.0f, cy = v * 2.0f - 1.0f;
         const float dx = (cx - c.sunX) * c.k, dy = (cy - c.sunY) * c.k;
-        float acc = tap<1>(a0, 0, c, u, v) * 0.5f;
-        float decay = 1.0f;
-        for (int i = 0; i < c.samples; i++) {
-            cx = cx - dx;
-            cy = cy - dy;
-            float s = tap<1>(a0, 0, c, cx * 0.5f + 0.5f, cy * 0.5f + 0.5f) * 0.5f;
-            s = s * (c.sw * decay);
-            acc = acc + s;
-            decay = decay * c.decay;
+        const At home = locate(m, u, v);
+        float acc = (m.use && all_lanes(inside(m, home)) ? tap_inside(a0, m, home) : tap_edge(a0, c, u, v)) * 0.5f;
+        float decay = 1.0f, sw = c.sw, fade = c.decay;
+        asm("" : "+v"(decay), "+v"(sw), "+v"(fade));
+        // Up to four taps at a time: they lie in order on a line, so if the outer two are inside, all are.
+        for (int i = 0; i < c.samples; i += 4) {
+            const int n = min(c.samples - i, 4);
+            float tu[4], tv[4], t[4];
+            At at[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                cx = cx - dx;
+                cy = cy - dy;
+                tu[k] = __builtin_fmaf(cx, 0.5f, 0.5f);
+                tv[k] = __builtin_fmaf(cy, 0.5f, 0.5f);
+                at[k] = locate(m, tu[k], tv[k]);
+            }
+            if (m.use && n == 4 && all_lanes(inside(m, at[0]) && inside(m, at[3]))) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) t[k] = tap_inside(a0, m, at[k]);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (k < n) t[k] = tap_edge(a0, c, tu[k], tv[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if (k >= n) break;
+                acc = acc + (t[k] * 0.5f) * (sw * decay);
+                decay = decay * fade;
+            }
         }
         a = acc * c.godExposure;
     }
     alpha[(uint32_t)y * (uint32_t)c.pitch + (uint32_t)x] = a;
 }
 
-__constant__ float kBlurTaps[10] = {-0.08f, -0.05f, -0.03f, -0.02f, -0.01f, 0.01f, 0.02f, 0.03f, 0.05f, 0.08f};
-
 __global__ __launch_bounds__(256) void blur_tonemap_kernel(const mm::PostConsts c, const float4* __restrict__ img,
                                                            const float* __restrict__ alpha, float4* __restrict__ hdr,
                                                            uint32_t* __restrict__ rgba8) {
     int x, y;
     if (!xcd_tile(c, x, y) || x >= c.width || y >= c.height) return;
-    const float u = __fdiv_rn((float)x + 0.5f, (float)c.width), v = __fdiv_rn((float)y + 0.5f, (float)c.height);
+    const Map m = make_map(c);
+    const float u = div_by((float)x + 0.5f, (float)c.width, c.rw), v = div_by((float)y + 0.5f, (float)c.height, c.rh);
     float rgb[3];
-    tap_rgb(img, c, u, v, rgb);
+    tap_rgb(img, c, m, u, v, rgb);
     float o[3] = {rgb[0], rgb[1], rgb[2]};
     if (!c.below) {
         const float sx = u * 2.0f - 1.0f, sy = v * 2.0f - 1.0f;
@@ -194,12 +299,29 @@ __global__ __launch_bounds__(256) void blur_tonemap_kernel(const mm::PostConsts 
         const float dist = sqrt_rn(lx * lx + ly * ly);
         lx = __fdiv_rn(lx, dist);
         ly = __fdiv_rn(ly, dist);
+        // taps -0.08 .. 0.08 along the line to the sun, in order: if the outer two are inside, all are
+        float scale = c.blurScale, gain = c.blurGain;
+        asm("" : "+v"(scale), "+v"(gain));
+        constexpr float kTaps[5] = {0.08f, 0.05f, 0.03f, 0.02f, 0.01f};
+        float tu[10], tv[10], t[10];
+#pragma unroll
+        for (int i = 0; i < 5; i++) {
+            const float ox = ((kTaps[i] * lx) * scale) * dist, oy = ((kTaps[i] * ly) * scale) * dist;
+            tu[i] = __builtin_fmaf(sx - ox, 0.5f, 0.5f);
+            tv[i] = __builtin_fmaf(sy - oy, 0.5f, 0.5f);
+            tu[9 - i] = __builtin_fmaf(sx + ox, 0.5f, 0.5f);
+            tv[9 - i] = __builtin_fmaf(sy + oy, 0.5f, 0.5f);
+        }
+        if (m.use && all_lanes(inside(m, locate(m, tu[0], tv[0])) && inside(m, locate(m, tu[9], tv[9])))) {
+#pragma unroll
+            for (int i = 0; i < 10; i++) t[i] = tap_inside(alpha, m, locate(m, tu[i], tv[i]));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 10; i++) t[i] = tap_edge(alpha, c, tu[i], tv[i]);
+        }
         float acc = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 10; i++) {
-            const float ox = ((kBlurTaps[i] * lx) * c.blurScale) * dist, oy = ((kBlurTaps[i] * ly) * c.blurScale) * dist;
-            acc = acc + tap<1>(alpha, 0, c, (sx + ox) * 0.5f + 0.5f, (sy + oy) * 0.5f + 0.5f) * c.blurGain;
-        }
+        for (int i = 0; i < 10; i++) acc = acc + t[i] * gain;
         acc = __fdiv_rn(acc, 10.0f);
         for (int k = 0; k < 3; k++) o[k] = c.gc[k] * acc + 0.5f * rgb[k];
     }
@@ -208,15 +330,33 @@ __global__ __launch_bounds__(256) void blur_tonemap_kernel(const mm::PostConsts 
     if (rgba8) {
         const float vx = u - 0.5f, vy = v - 0.5f;
         const float vig = vx * vx + vy * vy;
-        uint32_t q = 255u << 24;
+        // framebuffer 2 sampled at the pixel centre returns this pixel's radial-blur value
+        float t[3];
+        bool ok = true;
         for (int k = 0; k < 3; k++) {
-            // framebuffer 2 sampled at the pixel centre returns this pixel's radial-blur value
-            float t = uc2(c.exposure * o[k]);
-            t = t * c.whitemap;
-            t = exp2_series(c.invGamma * log2_series(t));  // pow (tonemap.frag:22)
-            t = t * (1.0f - vig) + c.vignette[k] * vig;
-            q |= unorm8(t) << (8 * k);
+            t[k] = c.exposure * o[k];
+            ok = ok && __float_as_uint(t[k]) <= __float_as_uint(1e9f);  // and not negative, not NaN
         }
+        if (all_lanes(ok)) {
+            for (int k = 0; k < 3; k++) t[k] = uc2<true>(t[k]) * c.whitemap;
+        } else {
+            for (int k = 0; k < 3; k++) t[k] = uc2<false>(t[k]) * c.whitemap;
+        }
+        ok = __builtin_amdgcn_classf(t[0], 0x100) && __builtin_amdgcn_classf(t[1], 0x100) &&
+             __builtin_amdgcn_classf(t[2], 0x100);  // positive normal numbers
+        if (all_lanes(ok)) {
+            for (int k = 0; k < 3; k++) t[k] = c.invGamma * log2_series<true>(t[k]);  // pow (tonemap.frag:22)
+        } else {
+            for (int k = 0; k < 3; k++) t[k] = c.invGamma * log2_series<false>(t[k]);
+        }
+        ok = fabsf(t[0]) < 126.0f && fabsf(t[1]) < 126.0f && fabsf(t[2]) < 126.0f;
+        if (all_lanes(ok)) {
+            for (int k = 0; k < 3; k++) t[k] = exp2_series<true>(t[k]);
+        } else {
+            for (int k = 0; k < 3; k++) t[k] = exp2_series<false>(t[k]);
+        }
+        uint32_t q = 255u << 24;
+        for (int k = 0; k < 3; k++) q |= unorm8(t[k] * (1.0f - vig) + c.vignette[k] * vig) << (8 * k);
         rgba8[i] = q;
     }
 }
