@@ -920,11 +920,13 @@ int mm_post_process(const mm_camera_ubo* camera, const mm_sun_ubo* sun, const fl
     c.sunY = sp[1] / sp[3];
     c.width = width;
     c.height = height;
-    {
-        // exact for every t < tiles while tiles * gx < 2^32 (the magic number is at most gx / 2^32 too large)
-        const unsigned long long gx = ((unsigned long long)width + 15) / 16, tiles = gx * (((unsigned long long)height + 15) / 16);
-        c.tileMagic = gx > 1 && tiles * gx < (1ull << 32) ? (uint32_t)(((1ull << 32) + gx - 1) / gx) : 0u;
-    }
+    // exact for every t < tiles while tiles * gx < 2^32 (the magic number is at most gx / 2^32 too large)
+    auto magic = [&](unsigned long long gx) {
+        const unsigned long long tiles = gx * (((unsigned long long)height + 15) / 16);
+        return gx > 1 && tiles * gx < (1ull << 32) ? (uint32_t)(((1ull << 32) + gx - 1) / gx) : 0u;
+    };
+    c.tileMagic = magic(((unsigned long long)width + 15) / 16);
+    c.wideTileMagic = magic(((unsigned long long)width + 63) / 64);
     c.rw = 1.0f / (float)width;
     c.rh = 1.0f / (float)height;
     c.pitch = row_pitch_px;

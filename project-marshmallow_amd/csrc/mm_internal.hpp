@@ -117,7 +117,7 @@ int launch_shadow(int fset, const ShadowConsts& c, const TexView& weather, const
 // Constants of one post-chain pass (god-ray.frag, radialBlur.frag, tonemap.frag), derived on the host.
 struct PostConsts {
     int width, height, pitch, bits, samples, below;
-    uint32_t tileMagic;           // ceil(2^32 / tiles a row): umulhi(t, it) = t / that row; 0: divide
+    uint32_t tileMagic, wideTileMagic;  // ceil(2^32 / n), n tiles of 16 / 64 pixels a row: umulhi(t, it) = t / n; 0: divide
     float rw, rh;                 // 1 / width, 1 / height
     float sunX, sunY;             // the sun in NDC: ((proj * view) * location).xy / w
     float k;                      // (1 / samples) * density

@@ -1,9 +1,10 @@
 // Post chain for gfx950: the HIP counterpart of the offscreen passes that consume the cloud image,
 // god-ray.frag:41-76 -> radialBlur.frag:36-63 -> tonemap.frag:11-34 (VulkanApplication.cpp:938-966).
 //
-// Three launches of 16x16-pixel blocks (four wave64 rows of 16x4), one contiguous band of tiles per XCD:
+// Three launches of blocks of 256 work-items (16x16 pixels; 64x16 for the god rays), one contiguous band of
+// tiles per XCD:
 //   alpha_plane_kernel  the cloud image's alpha as a plane of floats (16 B read, 4 B written);
-//   god_ray_kernel      one work-item per pixel: 9 bilinear taps of that plane (centre + 8 toward
+//   god_ray_kernel      four pixels a work-item: 9 bilinear taps of that plane each (centre + 8 toward
 //                       the sun), writes the alpha plane of framebuffer 1 (4 B/pixel);
 //   blur_tonemap_kernel one work-item per pixel: bilinear centre tap of the image's RGB, 10 bilinear
 //                       taps of that alpha plane toward the sun, the radial-blur colour, then the
@@ -14,7 +15,7 @@
 // read + 4 (or 20) B written (radial blur + tonemap) per pixel. The tap kernels are bound by vector operations
 // and by the caches' lanes: waves whose taps are all inside the image take a tap without clamps and with one
 // 8-byte load a row, and the tonemap of ordinary numbers takes unscaled divisions and no special cases
-// (1080p with the HDR output: god rays 29 us -> 22, blur + tonemap 51 -> 38, the chain 78 -> 62).
+// (1080p with the HDR output: god rays 29 us -> 17, blur + tonemap 51 -> 38, the chain 78 -> 56).
 // Arithmetic follows the shaders' evaluation order with IEEE division/sqrt and no contraction; the
 // sampler and the other choices GLSL leaves open are the scalar restatement's, so the result is the
 // same bit for bit.
@@ -113,6 +114,15 @@ __device__ __forceinline__ float tap_inside(const float* __restrict__ img, const
     return lerp_r(lerp_r(p.l, p.r, fx), lerp_r(q.l, q.r, fx), fy);
 }
 
+// One row of tap_inside: two neighbouring texels `off` bytes into a line.
+__device__ __forceinline__ float row_filter(const float* __restrict__ line, uint32_t off, float fx) {
+    struct __attribute__((packed, aligned(4))) Pair {
+        float l, r;
+    };
+    const Pair p = *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(line) + off);
+    return lerp_r(p.l, p.r, fx);
+}
+
 // The RGB of one bilinear tap of the RGBA image (one 16-byte load per texel).
 __device__ __forceinline__ void lerp_rgb(const float4& t00, const float4& t01, const float4& t10, const float4& t11,
                                          float fx, float fy, float rgb[3]) {
@@ -206,20 +216,28 @@ __device__ __forceinline__ float exp2_series(float t) {
     return __builtin_amdgcn_ldexpf(p * 1.41421356f, (int)n);
 }
 
-// Block -> 16x16 tile. Workgroups are dealt round-robin to the 8 XCDs (block b runs on XCD b mod 8),
+// Block -> tile. Workgroups are dealt round-robin to the 8 XCDs (block b runs on XCD b mod 8),
 // each with its own L2; the taps of a pixel reach far toward the sun, so tiles that share cache
 // lines should share an XCD. Block b takes tile (b mod 8) * per + b / 8 of the row-major tile list
 // (per = ceil(tiles / 8)): each XCD marches one contiguous band of tile rows. Returns false for the
 // padding blocks past the last tile.
-__device__ __forceinline__ bool xcd_tile(const mm::PostConsts& c, int& x, int& y) {
-    const int gx = (c.width + 15) >> 4, tiles = gx * ((c.height + 15) >> 4);
+__device__ __forceinline__ bool xcd_tile(const mm::PostConsts& c, int widthLog2, int heightLog2, uint32_t magic, int& x,
+                                         int& y) {
+    const int gx = (c.width + (1 << widthLog2) - 1) >> widthLog2;
+    const int tiles = gx * ((c.height + (1 << heightLog2) - 1) >> heightLog2);
     const int per = (tiles + 7) >> 3;
     const int t = (int)(blockIdx.x & 7u) * per + (int)(blockIdx.x >> 3);
     if (t >= tiles) return false;
-    const int row = c.tileMagic ? (int)__umulhi((uint32_t)t, c.tileMagic) : t / gx;  // scalar multiply
-    x = (t - row * gx) * 16 + (threadIdx.x & 15);
-    y = row * 16 + (threadIdx.x >> 4);
+    const int row = magic ? (int)__umulhi((uint32_t)t, magic) : t / gx;  // scalar multiply
+    x = (t - row * gx) << widthLog2;
+    y = row << heightLog2;
     return true;
+}
+__device__ __forceinline__ bool pixel_16x16(const mm::PostConsts& c, int& x, int& y) {
+    if (!xcd_tile(c, 4, 4, c.tileMagic, x, y)) return false;
+    x += threadIdx.x & 15;
+    y += threadIdx.x >> 4;
+    return x < c.width && y < c.height;
 }
 
 __device__ __forceinline__ uint32_t unorm8(float v) {
@@ -231,63 +249,140 @@ __device__ __forceinline__ uint32_t unorm8(float v) {
 __global__ __launch_bounds__(256) void alpha_plane_kernel(const mm::PostConsts c, const float4* __restrict__ img,
                                                           float* __restrict__ plane) {
     int x, y;
-    if (!xcd_tile(c, x, y) || x >= c.width || y >= c.height) return;
+    if (!pixel_16x16(c, x, y)) return;
     const uint32_t i = (uint32_t)y * (uint32_t)c.pitch + (uint32_t)x;
     plane[i] = img[i].w;
 }
 
+// A wave takes 64 columns of R rows, R pixels a lane. A tap's x depends on the column alone and its y on the row
+// alone: a lane's pixels share the x, and the rows' y are computed by lanes 0 .. R - 1 (lane mod R) and read back
+// as scalars. The R footprints of a tap together cover at most R + 1 rows of texels as long as the rows' taps
+// are no farther apart than the rows are (any density up to 1): for R = 4 five 8-byte loads and five horizontal
+// filters instead of eight. One pixel a lane of a 16x4 wave was bound by the L1's four lanes a cycle: 22 us at
+// 1080p for the nine taps, 17 with R = 4. Images under a million pixels leave the chip idle and wait for their
+// loads instead: R = 1 and three taps in flight (the chain, us, at R = 1 / R = 4: 640x360 16.2 / 19.3, 960x540
+// 23.4 / 25.0, 1280x720 34.0 / 33.4, 1600x900 47.8 / 43.7, 1920x1080 62.9 / 58.0; R = 4 with three taps: 59.8).
+template <int N>
+struct Count {
+    static constexpr int value = N;
+};
+template <int RL, int BATCH>
 __global__ __launch_bounds__(256) void god_ray_kernel(const mm::PostConsts c, const float* __restrict__ a0,
                                                       float* __restrict__ alpha) {
+    constexpr int R = 1 << RL;
     int x, y;
-    if (!xcd_tile(c, x, y) || x >= c.width || y >= c.height) return;
-    float a = 1.0f;  // sun below the horizon: the pass writes alpha 1 (god-ray.frag:55-57)
+    if (!xcd_tile(c, 6, 2 + RL, RL == 2 ? c.wideTileMagic : 0u, x, y)) return;
+    const int lane = (int)(threadIdx.x & 63u);
+    const int col = x + lane, row = y + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * R;
+    if (row >= c.height) return;  // the whole wave: every lane stays to the end for the scalars
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = 1.0f;  // sun below the horizon: the pass writes alpha 1 (god-ray.frag:55-57)
     if (!c.below) {
         const Map m = make_map(c);
-        const float u = div_by((float)x + 0.5f, (float)c.width, c.rw), v = div_by((float)y + 0.5f, (float)c.height, c.rh);
+        const float u = div_by((float)min(col, c.width - 1) + 0.5f, (float)c.width, c.rw);
+        const float v = div_by((float)min(row + (lane & (R - 1)), c.height - 1) + 0.5f, (float)c.height, c.rh);
         float cx = u * 2.0f - 1.0f, cy = v * 2.0f - 1.0f;
         const float dx = (cx - c.sunX) * c.k, dy = (cy - c.sunY) * c.k;
-        const At home = locate(m, u, v);
-        float acc = (m.use && all_lanes(inside(m, home)) ? tap_inside(a0, m, home) : tap_edge(a0, c, u, v)) * 0.5f;
         float decay = 1.0f, sw = c.sw, fade = c.decay;
         asm("" : "+v"(decay), "+v"(sw), "+v"(fade));
-        // Up to four taps at a time: they lie in order on a line, so if the outer two are inside, all are.
-        for (int i = 0; i < c.samples; i += 4) {
-            const int n = min(c.samples - i, 4);
-            float tu[4], tv[4], t[4];
-            At at[4];
+        // N taps from tap i on (-1: the pixel's own), their loads in flight together. The taps lie in order on a
+        // line: if the outer two are inside, all are.
+        auto taps = [&](auto count, int i) {
+            constexpr int N = decltype(count)::value;
+            float tu[N], tv[N], t[N][R];
+            At a[N];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                cx = cx - dx;
-                cy = cy - dy;
-                tu[k] = __builtin_fmaf(cx, 0.5f, 0.5f);
-                tv[k] = __builtin_fmaf(cy, 0.5f, 0.5f);
-                at[k] = locate(m, tu[k], tv[k]);
+            for (int k = 0; k < N; k++) {
+                tu[k] = u;
+                tv[k] = v;
+                if (i + k >= 0) {
+                    cx = cx - dx;
+                    cy = cy - dy;
+                    tu[k] = __builtin_fmaf(cx, 0.5f, 0.5f);
+                    tv[k] = __builtin_fmaf(cy, 0.5f, 0.5f);
+                }
+                a[k] = locate(m, tu[k], tv[k]);
             }
-            if (m.use && n == 4 && all_lanes(inside(m, at[0]) && inside(m, at[3]))) {
+            if (m.use && all_lanes(inside(m, a[0]) && (N == 1 || inside(m, a[N - 1])))) {
+                int iy[N][R];
+                uint32_t off[N];
+                float fx[N], fy[N][R];
+                bool near = true;
 #pragma unroll
-                for (int k = 0; k < 4; k++) t[k] = tap_inside(a0, m, at[k]);
+                for (int k = 0; k < N; k++) {
+                    int kx, ky;
+                    float f;
+                    texel(a[k], kx, ky, fx[k], f);
+                    off[k] = ((uint32_t)kx >> 6) & ~3u;
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        iy[k][r] = __builtin_amdgcn_readlane(ky, r) >> 8;
+                        fy[k][r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), r));
+                        if (r > 0) near = near && (unsigned)(iy[k][r] - iy[k][r - 1]) <= 1u;
+                    }
+                }
+                if (near) {
+                    float h[N][R + 1];
+#pragma unroll
+                    for (int k = 0; k < N; k++)
+#pragma unroll
+                        for (int r = 0; r <= R; r++)  // rows past the last footprint are read as the last row, unused
+                            h[k][r] = row_filter(a0 + (size_t)(uint32_t)min(iy[k][0] + r, c.height - 1) * (uint32_t)c.pitch,
+                                                 off[k], fx[k]);
+#pragma unroll
+                    for (int k = 0; k < N; k++)
+#pragma unroll
+                        for (int r = 0; r < R; r++) {
+                            if (r > 0 && iy[k][r] != iy[k][r > 0 ? r - 1 : 0]) {
+#pragma unroll
+                                for (int l = 0; l + r <= R; l++) h[k][l] = h[k][l + 1];
+                            }
+                            t[k][r] = lerp_r(h[k][0], h[k][1], fy[k][r]);
+                        }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < N; k++)
+#pragma unroll
+                        for (int r = 0; r < R; r++) {
+                            const float* line = a0 + (size_t)(uint32_t)iy[k][r] * (uint32_t)c.pitch;
+                            t[k][r] = lerp_r(row_filter(line, off[k], fx[k]), row_filter(line + c.pitch, off[k], fx[k]),
+                                             fy[k][r]);
+                        }
+                }
             } else {
 #pragma unroll
-                for (int k = 0; k < 4; k++)
-                    if (k < n) t[k] = tap_edge(a0, c, tu[k], tv[k]);
+                for (int k = 0; k < N; k++)
+#pragma unroll
+                    for (int r = 0; r < R; r++)
+                        t[k][r] = tap_edge(a0, c, tu[k], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tv[k]), r)));
             }
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                if (k >= n) break;
-                acc = acc + (t[k] * 0.5f) * (sw * decay);
-                decay = decay * fade;
+            for (int k = 0; k < N; k++) {
+                const float w = sw * decay;
+#pragma unroll
+                for (int r = 0; r < R; r++) acc[r] = i + k < 0 ? t[k][r] * 0.5f : acc[r] + (t[k][r] * 0.5f) * w;
+                if (i + k >= 0) decay = decay * fade;
             }
-        }
-        a = acc * c.godExposure;
+        };
+        int i = -1;
+        if constexpr (BATCH > 1)
+            for (; i + BATCH <= c.samples; i += BATCH) taps(Count<BATCH>{}, i);
+        for (; i < c.samples; i++) taps(Count<1>{}, i);
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r] = acc[r] * c.godExposure;
     }
-    alpha[(uint32_t)y * (uint32_t)c.pitch + (uint32_t)x] = a;
+    if (col >= c.width) return;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        if (row + r < c.height) alpha[(uint32_t)(row + r) * (uint32_t)c.pitch + (uint32_t)col] = acc[r];
 }
 
 __global__ __launch_bounds__(256) void blur_tonemap_kernel(const mm::PostConsts c, const float4* __restrict__ img,
                                                            const float* __restrict__ alpha, float4* __restrict__ hdr,
                                                            uint32_t* __restrict__ rgba8) {
     int x, y;
-    if (!xcd_tile(c, x, y) || x >= c.width || y >= c.height) return;
+    if (!pixel_16x16(c, x, y)) return;
     const Map m = make_map(c);
     const float u = div_by((float)x + 0.5f, (float)c.width, c.rw), v = div_by((float)y + 0.5f, (float)c.height, c.rh);
     float rgb[3];
@@ -296,9 +391,19 @@ __global__ __launch_bounds__(256) void blur_tonemap_kernel(const mm::PostConsts 
     if (!c.below) {
         const float sx = u * 2.0f - 1.0f, sy = v * 2.0f - 1.0f;
         float lx = c.sunX - sx, ly = c.sunY - sy;
-        const float dist = sqrt_rn(lx * lx + ly * ly);
-        lx = __fdiv_rn(lx, dist);
-        ly = __fdiv_rn(ly, dist);
+        const float d2 = lx * lx + ly * ly;
+        float dist;
+        if (all_lanes(fminf(fabsf(lx), fabsf(ly)) >= 0x1p-40f && d2 <= 0x1p80f)) {  // quotients far from subnormal
+            const float y = __builtin_amdgcn_rsqf(d2);
+            dist = sqrt_from_rsq(d2, y);
+            const float r = rcp_refine(dist, y);
+            lx = div_by(lx, dist, r);
+            ly = div_by(ly, dist, r);
+        } else {
+            dist = sqrt_rn(d2);
+            lx = __fdiv_rn(lx, dist);
+            ly = __fdiv_rn(ly, dist);
+        }
         // taps -0.08 .. 0.08 along the line to the sun, in order: if the outer two are inside, all are
         float scale = c.blurScale, gain = c.blurGain;
         asm("" : "+v"(scale), "+v"(gain));
@@ -373,7 +478,12 @@ int launch_post(const PostConsts& c, const float* image, float* scratch, float* 
     float* a0 = scratch;
     float* a1 = scratch + (size_t)c.pitch * c.height;
     if (!c.below) hipLaunchKernelGGL(alpha_plane_kernel, grid, block, 0, s, c, (const float4*)image, a0);
-    hipLaunchKernelGGL(god_ray_kernel, grid, block, 0, s, c, (const float*)a0, a1);
+    const bool large = (long)c.width * c.height >= 1 << 20;  // see god_ray_kernel
+    const int rows = large ? 16 : 4;
+    const long wide = (long)((c.width + 63) / 64) * ((c.height + rows - 1) / rows);
+    const dim3 wideGrid((unsigned)(8 * ((wide + 7) / 8)));
+    if (large) hipLaunchKernelGGL((god_ray_kernel<2, 1>), wideGrid, block, 0, s, c, (const float*)a0, a1);
+    else hipLaunchKernelGGL((god_ray_kernel<0, 3>), wideGrid, block, 0, s, c, (const float*)a0, a1);
     hipLaunchKernelGGL(blur_tonemap_kernel, grid, block, 0, s, c, (const float4*)image, (const float*)a1,
                        (float4*)hdr, (uint32_t*)rgba8);
     return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
