@@ -289,11 +289,11 @@ def lanes_and_tiles(args):
         return 1, args.tile_width or 8
     rays = getattr(args, "width", 1920) * getattr(args, "height", 1080)
     if args.no_schedule:
-        lanes = args.lanes_per_ray or (8 if rays <= 400_000 else 2)
+        lanes = args.lanes_per_ray or (16 if rays <= 45_000 else 8 if rays <= 400_000 else 2)
     else:
-        lanes = args.lanes_per_ray or (8 if rays <= 200_000 else 4 if rays <= 480_000 else 2 if rays <= 1 << 20 else 1)
+        lanes = args.lanes_per_ray or (16 if rays <= 45_000 else 8 if rays <= 200_000 else 4 if rays <= 480_000 else 2 if rays <= 1 << 20 else 1)
     if lanes > 1:
-        return lanes, 8
+        return lanes, 4 if lanes == 16 else 8
     return 1, args.tile_width or (8 if args.no_schedule else 16)
 
 

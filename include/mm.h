@@ -217,7 +217,7 @@ typedef struct mm_march_params {
                                    the image does not depend on it */
     int32_t lanes_per_ray;      /* 1, 2, 4 or 8 lanes march one ray, sampling the next trips ahead
                                    and committing them in order (0 = default, by the rays marched:
-                                   8 for a phase of up to 2^19 rays and a frame of up to 400 000, else
+                                   16 up to 45 000 of them, 8 for a phase of up to 2^19 rays and a frame of up to 400 000, else
                                    2; through a schedule 8, 4, 2 and 1 from the smallest frames to
                                    those over 2^20 rays); plain cones only (the surrogate-lit march
                                    takes at most 2, other modes 1); the image does not depend on it */

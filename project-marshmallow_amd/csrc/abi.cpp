@@ -285,6 +285,9 @@ struct CollectArgs {
 //     230 400: 839 491 269 247 / 573 335 209 247;  518 400: 785 459 420 473 / 622 384 394 506;
 //     921 600: 807 641 712 820 / 681 616 653 872;  1 440 000: 915 964 1087 1268 / 853 913 985 1341
 //   one phase  518 400: 826 600 549 459 / 613 401 475 467;  921 600: 1137 684 855 841 / 875 617 727 874
+// 16 lanes pay for both scenes up to 45 000 rays or so, 8 and 16 lanes: 16 384 rays 121 77 / 84 63; one phase
+//   32 400: 140 92 / 104 83;  57 600: 147 111 / 107 120;  65 536: 141 112 / 110 132.
+constexpr long long kRays16 = 45000;
 constexpr long long kFrameRays8 = 400000, kPhaseRays8 = 1 << 19;
 constexpr long long kScheduledRays8 = 200000, kScheduledRays4 = 480000, kScheduledRays2 = 1 << 20;
 // A views launch has many more waves (64 views of 256x256 to 1920x1080: 33.6 M pixels, 1 / 2 / 4
@@ -300,7 +303,7 @@ constexpr int kDefaultViewsTileWidth = 16;
 static void horizon_first_rows(mm::MarchConsts& c) {
     c.rowStart = 0;
     c.rowDir = 1;
-    const int th = c.lanesPerRay > 1 ? 64 / c.lanesPerRay / 8 : (64 >> c.tileShift);
+    const int th = (64 / c.lanesPerRay) >> c.tileShift;
     auto up = [&](int tr) {  // y of the unnormalised ray direction at the tile row's middle
         int gj = tr * th + th / 2;
         if (gj > c.gridH - 1) gj = c.gridH - 1;
@@ -489,6 +492,9 @@ struct mm_march_schedule {
     int device = 0;
 };
 
+// The ray-parallel kernel's tiles: 8 x (8 / lanes) rays, 4 x 1 with 16 lanes.
+static int tile_shift(int lanes) { return lanes == 16 ? 2 : 3; }
+
 // Lanes per ray of a march (params.lanes_per_ray; 0 = by the rays, see kFrameRays8); 1 for the other cone
 // modes and the lock-step kernel. A schedule takes no more lanes than its record holds the tiles of (the
 // one-lane tiles are the fewest). The image does not depend on it.
@@ -498,15 +504,16 @@ static int lanes_for(const mm::MarchConsts& c, const mm_march_params* params, in
     const bool one_phase = phase >= 0 || phase == MM_PHASE_FROM_UBO;
     if (lpr == 0) {
         const long long rays = (long long)c.gridW * c.gridH;
-        if (one_phase) {
-            lpr = sched || rays <= kPhaseRays8 ? 8 : 2;
-        } else if (!sched) {
-            lpr = rays <= kFrameRays8 ? 8 : 2;
-        } else {
-            lpr = rays <= kScheduledRays8 ? 8 : rays <= kScheduledRays4 ? 4 : rays <= kScheduledRays2 ? 2 : 1;
-            while (lpr > 1 && ((c.gridW + 7) / 8) * (long long)((c.gridH + 8 / lpr - 1) / (8 / lpr)) > sched->capacity)
-                lpr /= 2;
-        }
+        if (one_phase) lpr = sched || rays <= kPhaseRays8 ? 8 : 2;
+        else if (!sched) lpr = rays <= kFrameRays8 ? 8 : 2;
+        else lpr = rays <= kScheduledRays8 ? 8 : rays <= kScheduledRays4 ? 4 : rays <= kScheduledRays2 ? 2 : 1;
+        if (rays <= kRays16) lpr = 16;
+        auto tiles = [&](int lanes) {
+            const int shift = tile_shift(lanes), th = (64 / lanes) >> shift;
+            return (long long)((c.gridW + (1 << shift) - 1) >> shift) * ((c.gridH + th - 1) / th);
+        };
+        if (sched)
+            while (lpr > (one_phase ? 8 : 1) && tiles(lpr) > sched->capacity) lpr /= 2;
     }
     if (c.flags & MM_MARCH_NO_BATCH) return 1;
     // the surrogate-lit march runs with one or two lanes per ray; the sample recorder with one
@@ -515,14 +522,13 @@ static int lanes_for(const mm::MarchConsts& c, const mm_march_params* params, in
     return lpr;
 }
 
-// The ray-parallel kernel's tiles of 8 x (8 / lanes) rays (lanes 1 keeps the 64-ray tiles) and the
-// launch order of their rows.
+// The ray-parallel kernel's tiles (lanes 1 keeps the 64-ray tiles) and the launch order of their rows.
 static void set_lanes(mm::MarchConsts& c, int lpr) {
     c.lanesPerRay = lpr;
     if (lpr > 1) {
-        const int th = 64 / lpr / 8;
-        c.tileShift = 3;
-        c.tilesX = (c.gridW + 7) >> 3;
+        c.tileShift = tile_shift(lpr);
+        const int th = (64 / lpr) >> c.tileShift;
+        c.tilesX = (c.gridW + (1 << c.tileShift) - 1) >> c.tileShift;
         c.tilesY = (c.gridH + th - 1) / th;
         c.tiles = c.tilesX * c.tilesY;
     }

@@ -1406,7 +1406,7 @@ void march_batched_kernel(const MarchConsts c, const MarchTextures tx,
 }
 
 // ---------------------------------------------------------------- ray-parallel march
-// LPR lanes per ray (2, 4 or 8), 64 / LPR rays per wave in an 8-wide tile. Every lane of a ray holds
+// LPR lanes per ray (2, 4, 8 or 16), 64 / LPR rays per wave in a tile 8 wide (4 with 16 lanes). Every lane of a ray holds
 // the ray's whole state. Each loop round, lane k of the ray samples trip k ahead: at t plus k times
 // the step (the same float additions the loop makes), in the current mode. The ray's lanes then
 // commit the trips up to the first whose mode, step or t no longer match what was sampled (a mode switch or
@@ -1507,13 +1507,13 @@ template <int FSET, bool COUNT, int LPR, int MODE = CONE_PLAIN>
 __device__ __forceinline__ void march_rp_tile(const MarchConsts& c, const MarchTextures& tx, const int tile,
                                               float* __restrict__ out, unsigned long long* __restrict__ counts,
                                               CostRec costRec) {
-    static_assert(LPR == 2 || LPR == 4 || LPR == 8, "lanes per ray");
-    constexpr int TH = 64 / LPR / 8;  // tile: 8 x TH rays
+    static_assert(LPR == 2 || LPR == 4 || LPR == 8 || LPR == 16, "lanes per ray");
+    constexpr int TW = LPR == 16 ? 4 : 8, TH = 64 / LPR / TW;  // tile: TW x TH rays
     __shared__ typename ConeQueueOf<MODE>::type q;
     const int lane = threadIdx.x, ray = lane / LPR, k = lane % LPR, first = lane - k;
     // tile: physical tile index (row x tilesX + column)
-    const int gi = (tile % c.tilesX) * 8 + (ray & 7);
-    const int gj = (tile / c.tilesX) * TH + (ray >> 3);
+    const int gi = (tile % c.tilesX) * TW + (ray & (TW - 1));
+    const int gj = (tile / c.tilesX) * TH + ray / TW;
     const bool valid = gi < c.gridW && gj < c.gridH;
     int px = 0, py = 0;
     if (valid) tile_pixel(c, gi, gj, px, py);
@@ -1801,6 +1801,8 @@ int launch_t(const MarchConsts& c, const MarchTextures& t, float* out, unsigned 
     dim3 grid((unsigned)c.tiles), block(64);
     if (c.coneMode == CONE_PLAIN && (c.flags & MM_MARCH_NO_BATCH))
         hipLaunchKernelGGL((march_kernel<FSET, COUNT>), grid, block, 0, s, c, t, out, counts);
+    else if (c.coneMode == CONE_PLAIN && c.lanesPerRay == 16)
+        hipLaunchKernelGGL((march_rp_kernel<FSET, COUNT, 16>), grid, block, 0, s, c, t, out, counts);
     else if (c.coneMode == CONE_PLAIN && c.lanesPerRay == 8)
         hipLaunchKernelGGL((march_rp_kernel<FSET, COUNT, 8>), grid, block, 0, s, c, t, out, counts);
     else if (c.coneMode == CONE_PLAIN && c.lanesPerRay == 4)
