@@ -169,7 +169,9 @@ __global__ void pack_kernel(const float* __restrict__ p, uint4* __restrict__ fra
 // A step is bound by latency, not by its 15 MFLOP: 64 workgroups at the configured batch, each a chain of about
 // 75 MFMAs per wave. One wave per 64 rows with the gradients added by atomics from every 32-row tile (2.4 M
 // device-scope atomics a step) and separate clearing, Adam and packing launches took 146 us a step; this takes
-// 11.5 us and the update 4. The gradient of 500 000 rows: 6.4 ms before, 0.19 ms. The weights go through LDS once
+// 11.5 us and the update 4. The gradient of a million rows: 12.5 ms before, 0.16 ms
+// (0.26 with the workgroups' atomics in MFMA order, a cache line each, instead of through LDS; of 30 000 rows 112
+// us against 24). The weights go through LDS once
 // per workgroup: each wave loading its own fragments into registers took 15.7 us (144 of them, the rest in
 // accumulator registers at a move per use).
 constexpr int kTrainRows = 128, kTrainWaves = kTrainRows / 32;
@@ -188,19 +190,8 @@ struct alignas(16) TrainLds {
     float red[kTrainWaves][3];
 };
 
-// Gradient sink: a workgroup's own partial buffer (plain stores) or a shared buffer (atomics).
-template <bool ATOMIC>
-__device__ __forceinline__ void put(float* g, int i, float v) {
-    if (ATOMIC) atomicAdd(&g[i], v);
-    else g[i] = v;
-}
-template <bool ATOMIC>
 __device__ __forceinline__ void put4(float* g, int i, const f32x16& a, int r) {  // i a multiple of 4
-    if (ATOMIC) {
-        for (int k = 0; k < 4; k++) atomicAdd(&g[i + k], a[r + k]);
-    } else {
-        *reinterpret_cast<float4*>(g + i) = make_float4(a[r], a[r + 1], a[r + 2], a[r + 3]);
-    }
+    *reinterpret_cast<float4*>(g + i) = make_float4(a[r], a[r + 1], a[r + 2], a[r + 3]);
 }
 
 // Rows: hashed draws from the n samples (`rows` = the batch) by the model's step counter plus `step`, or, with
@@ -348,7 +339,9 @@ __global__ __launch_bounds__(64 * kTrainWaves, 1) void train_kernel(
             }
         __syncthreads();  // the next rows overwrite the tiles
     }
-    float* g = ATOMIC ? out : out + (size_t)blockIdx.x * kPartial;
+    // ATOMIC: put together in LDS (the tiles are no longer read), then added in order, 64 neighbours at a time
+    static_assert(sizeof(TrainLds::act) >= sizeof(float) * kPartial, "the gradients take the activations' place");
+    float* g = ATOMIC ? reinterpret_cast<float*>(&L.act) : out + (size_t)blockIdx.x * kPartial;
     // loss and output biases: summed over the wave, then over the four waves
     for (int off = 32; off > 0; off >>= 1) {
         lossv += __shfl_xor(lossv, off);
@@ -364,26 +357,29 @@ __global__ __launch_bounds__(64 * kTrainWaves, 1) void train_kernel(
     if (threadIdx.x < 3) {
         float s = 0.0f;
         for (int k = 0; k < kTrainWaves; k++) s += L.red[k][threadIdx.x];
-        if (threadIdx.x == 0) put<ATOMIC>(ATOMIC ? loss : g, ATOMIC ? 0 : kParams, s);
-        else put<ATOMIC>(g, oB4 + (int)threadIdx.x - 1, s);
+        g[threadIdx.x == 0 ? kParams : oB4 + (int)threadIdx.x - 1] = s;
     }
     const int mt = w >> 1, nt = w & 1;
 #pragma unroll
     for (int r = 0; r < 16; r += 4) {
         const int u = 2 * r + 4 * h;  // crow(r, h)
-        put4<ATOMIC>(g, oW3 + (32 * nt + c) * kHidden + 32 * mt + u, acc[0], r);
-        put4<ATOMIC>(g, oW2 + (32 * nt + c) * kHidden + 32 * mt + u, acc[1], r);
+        put4(g, oW3 + (32 * nt + c) * kHidden + 32 * mt + u, acc[0], r);
+        put4(g, oW2 + (32 * nt + c) * kHidden + 32 * mt + u, acc[1], r);
         if (w < 2) {
-            if (c < kIn) put4<ATOMIC>(g, oW1 + c * kHidden + 32 * nt + u, acc[2], r);
-            if (c == kIn) put4<ATOMIC>(g, oB1 + 32 * nt + u, acc[2], r);
-            if (c == 0) put4<ATOMIC>(g, oB2 + 32 * nt + u, acc[3], r);
+            if (c < kIn) put4(g, oW1 + c * kHidden + 32 * nt + u, acc[2], r);
+            if (c == kIn) put4(g, oB1 + 32 * nt + u, acc[2], r);
+            if (c == 0) put4(g, oB2 + 32 * nt + u, acc[3], r);
         } else if (c == 0) {
-            put4<ATOMIC>(g, oB3 + 32 * nt + u, acc[2], r);
+            put4(g, oB3 + 32 * nt + u, acc[2], r);
         }
     }
     if (w >= 2 && h == 0) {
-        put<ATOMIC>(g, oW4 + (32 * nt + c) * kOut, acc[3][0]);
-        put<ATOMIC>(g, oW4 + (32 * nt + c) * kOut + 1, acc[3][1]);
+        g[oW4 + (32 * nt + c) * kOut] = acc[3][0];
+        g[oW4 + (32 * nt + c) * kOut + 1] = acc[3][1];
+    }
+    if constexpr (ATOMIC) {
+        __syncthreads();
+        for (int i = (int)threadIdx.x; i <= kParams; i += 64 * kTrainWaves) atomicAdd(i < kParams ? out + i : loss, g[i]);
     }
 }
 
@@ -469,9 +465,10 @@ __global__ __launch_bounds__(256) void update_kernel(const float* __restrict__ p
 
 __global__ void advance_kernel(int* counter, int steps) { *counter += steps; }
 
-__global__ void zero_kernel(float* p, int n) {
+__global__ void zero_kernel(float* p, int n, float* one) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0.0f;
+    if (i == 0 && one) *one = 0.0f;
 }
 
 // Batch inference with the march's FP16 path: 64 samples per wave; out[i] = (o0, softplus(o1)).
@@ -502,7 +499,7 @@ int surrogate_init(void* model, uint32_t seed, void* stream) {
     hipStream_t s = (hipStream_t)stream;
     ModelPtrs p = ptrs(model);
     hipLaunchKernelGGL(init_kernel, dim3(blocks(kParams, 256)), dim3(256), 0, s, p.params, p.m, p.v, p.stats, seed);
-    hipLaunchKernelGGL(zero_kernel, dim3(blocks(kParams, 256)), dim3(256), 0, s, p.grads, kParams);
+    hipLaunchKernelGGL(zero_kernel, dim3(blocks(kParams, 256)), dim3(256), 0, s, p.grads, kParams, nullptr);
     hipLaunchKernelGGL(pack_kernel, dim3(blocks(kPackThreads, 256)), dim3(256), 0, s, p.params, p.frags, p.hfrags);
     return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
 }
@@ -512,7 +509,7 @@ int surrogate_fit_stats(void* model, const float* samples, int n, int stride, vo
     ModelPtrs p = ptrs(model);
     double* acc = nullptr;
     if (hipMallocAsync((void**)&acc, sizeof(double) * 2 * kIn, s) != hipSuccess) return MM_E_DEVICE;
-    hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, s, (float*)acc, 4 * kIn);
+    hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, s, (float*)acc, 4 * kIn, nullptr);
     hipLaunchKernelGGL(stats_sum_kernel, dim3(256), dim3(64), 0, s, samples, n, stride, acc);
     hipLaunchKernelGGL(stats_final_kernel, dim3(1), dim3(64), 0, s, acc, n, p.stats);
     (void)hipFreeAsync(acc, s);
@@ -556,8 +553,7 @@ int surrogate_gradient(const void* model, const float* samples, int n, int strid
                        void* stream) {
     hipStream_t s = (hipStream_t)stream;
     ModelPtrs p = ptrs(const_cast<void*>(model));
-    hipLaunchKernelGGL(zero_kernel, dim3(blocks(kParams, 256)), dim3(256), 0, s, grad_out, kParams);
-    hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, s, loss_out, 1);
+    hipLaunchKernelGGL(zero_kernel, dim3(blocks(kParams, 256)), dim3(256), 0, s, grad_out, kParams, loss_out);
     const unsigned nb = std::min(blocks(n, kTrainRows), (unsigned)kMaxTrainBlocks);
     hipLaunchKernelGGL(train_kernel<true>, dim3(nb), dim3(64 * kTrainWaves), 0, s, samples, n, stride, p.params,
                        p.stats, p.frags, grad_out, loss_out, 0u, nullptr, 0, n, 1.0f / (float)n);
