@@ -251,7 +251,7 @@ int mm_generate_noise_noalloc(const mm_noise_params* p, const mm_noise_set* out,
         const int s = mm::static_scratch(&ws);
         if (s) return s;
     }
-    return mm::launch_generate(p, out, ws, stream, /*allow_side=*/false);
+    return mm::launch_generate(p, out, ws, stream);
 }
 
 int mm_pack_texture(int32_t kind, const mm_texture* src, const mm_texture* dst, void* stream) {

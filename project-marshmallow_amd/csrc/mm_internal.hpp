@@ -170,9 +170,7 @@ int launch_march(int fset, const MarchConsts& c, const MarchTextures& t, float* 
 int launch_tile_order(unsigned* sched, int n, int* order, void* stream);
 
 // Noise generation launchers.
-// allow_side = false keeps every generator on `stream` (no second stream is created or used)
-int launch_generate(const mm_noise_params* p, const mm_noise_set* out, void* workspace, void* stream,
-                    bool allow_side = true);
+int launch_generate(const mm_noise_params* p, const mm_noise_set* out, void* workspace, void* stream);
 size_t noise_workspace_bytes();
 size_t static_scratch_bytes();
 int static_scratch(void** ptr);

@@ -43,8 +43,8 @@ __device__ __forceinline__ double sin_poly(double x) {
 }
 
 // Also resets the min / max cells of the field kernel that follows (mm: 3 x (min, max), see f2ord).
-__global__ void curl_table_kernel(uint8_t* __restrict__ table, uint32_t* __restrict__ mm) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void curl_table_kernel(uint8_t* __restrict__ table, uint32_t* __restrict__ mm) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < 6) mm[i] = i & 1 ? 0u : 0xffffffffu;
     if (i >= kLat * kLat * kLat) return;
     const float x = (float)(i % kLat - kLatOff), y = (float)((i / kLat) % kLat - kLatOff),
@@ -124,17 +124,25 @@ __device__ __forceinline__ float ord2f(uint32_t u) {
 }
 
 // curlNoiseFBM (ImageUtils.cpp:130-169) + min/max. A chain of dependent FP64 lerps: latency bounds it, not the
-// arithmetic. A block takes 64 texels and six waves, one per partial derivative (two FBMs, eight Perlin
-// evaluations); the first wave combines them. 128^2: 19-24 us, against 53-60 with a work-item per texel (256
-// waves of 48 Perlin evaluations each on 1024 SIMDs).
+// arithmetic. A block takes 64 texels; its four waves share the six partial derivatives (two FBMs, eight Perlin
+// evaluations each) and the first combines them. With a work-item per texel 128^2 took 53-60 us (256 waves of 48
+// Perlin evaluations each on 1024 SIMDs).
 constexpr int kCurlTexels = 64;
-__global__ __launch_bounds__(6 * kCurlTexels) void curl_field_kernel(const uint8_t* __restrict__ tab, int dim,
-                                                                     float* __restrict__ field,
-                                                                     uint32_t* __restrict__ mm) {
-    __shared__ float part[6][kCurlTexels];
-    const int lane = threadIdx.x & 63, d = threadIdx.x >> 6, i = blockIdx.x * kCurlTexels + lane;
+struct CurlArgs {
+    uint8_t* table;
+    uint32_t* mm;
+    float* field;
+    int dim;
+};
+__device__ __forceinline__ void curl_field(const CurlArgs& g, int block, float* lds) {
+    float(*part)[kCurlTexels] = reinterpret_cast<float(*)[kCurlTexels]>(lds);  // [6]
+    const uint8_t* tab = g.table;
+    const int dim = g.dim, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = block * kCurlTexels + lane;
+    float* field = g.field;
+    uint32_t* mm = g.mm;
     const bool in = i < dim * dim;
-    if (in) {
+    for (int d = wave; d < 6; d += 4) {
+        if (!in) continue;
         const int row = i / dim, col = i % dim;
         const float px = (float)col / (float)dim, py = (float)row / (float)dim;
         const double eps = 0.0005;
@@ -153,7 +161,7 @@ __global__ __launch_bounds__(6 * kCurlTexels) void curl_field_kernel(const uint8
         part[d][lane] = central(fbm_ref(tab, a[0], a[1], a[2], 3.f, 4), fbm_ref(tab, b[0], b[1], b[2], 3.f, 4));
     }
     __syncthreads();
-    if (d != 0) return;
+    if (wave != 0) return;
     float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     if (in) {
         const float v[3] = {part[4][lane] - part[5][lane], part[2][lane] - part[3][lane], part[0][lane] - part[1][lane]};
@@ -258,6 +266,12 @@ struct LdsCells {
     }
 };
 
+// 1 - min(sqrt(d2), 1). Distances below 2^-48 give 1 like that bound's, so the root needs no special case: 30
+// issue cycles against 70, once per Worley level.
+__device__ __forceinline__ float inverted(float d2) {
+    return 1.0f - sqrt_rn_rsq(__builtin_amdgcn_fmed3f(d2, 0x1p-96f, 1.0f));
+}
+
 // A lower bound of fl((b - u)^2) over u in [0, 1], with the same roundings (each is monotone): no cell of a row
 // whose bounds in y and z sum to `best` or more can lower it, so the row is skipped and the minimum is the same.
 __device__ __forceinline__ float near_sq(float b) {
@@ -289,8 +303,7 @@ __device__ __forceinline__ float worley_at(float px, float py, float pz, int cel
             }
         }
     }
-    float d = sqrt_rn(best);
-    return 1.0f - (d < 1.0f ? d : 1.0f);
+    return inverted(best);
 }
 
 // worley_at over staged cells: the same arithmetic, each row of neighbours at constant offsets from its first.
@@ -316,8 +329,7 @@ __device__ __forceinline__ float worley_at(float px, float py, float pz, int cel
             }
         }
     }
-    const float d = sqrt_rn(best);
-    return 1.0f - (d < 1.0f ? d : 1.0f);
+    return inverted(best);
 }
 
 __constant__ float kGrad[12][3] = {{1, 1, 0}, {-1, 1, 0}, {1, -1, 0}, {-1, -1, 0}, {1, 0, 1},  {-1, 0, 1},
@@ -361,28 +373,21 @@ __device__ __forceinline__ float perlin_at(float px, float py, float pz, int per
     return lerp_(y0, y1, uz);
 }
 
-__device__ float value2(float px, float py, int period, uint32_t seed) {
-    float qx = px * (float)period, qy = py * (float)period;
-    float fx = floorf(qx), fy = floorf(qy);
-    float tx = qx - fx, ty = qy - fy;
-    int ix = (int)fx, iy = (int)fy;
-    float sx = (tx * tx) * (3.0f - 2.0f * tx), sy = (ty * ty) * (3.0f - 2.0f * ty);
-    float v[4];
-    for (int c = 0; c < 4; c++) {
-        uint32_t h0, h1, h2;
-        hash3((uint32_t)wrapi(ix + (c & 1), period), (uint32_t)wrapi(iy + (c >> 1), period), 0u, seed, h0, h1, h2);
-        v[c] = u01(h0);
-    }
-    return lerp_(lerp_(v[0], v[1], sx), lerp_(v[2], v[3], sx), sy);
+// The value at lattice point (x, y) of a periodic grid.
+__device__ __forceinline__ float value_at(int x, int y, int period, uint32_t seed) {
+    uint32_t h0, h1, h2;
+    hash3((uint32_t)wrapi(x, period), (uint32_t)wrapi(y, period), 0u, seed, h0, h1, h2);
+    return u01(h0);
 }
-
-__device__ float value_fbm(float px, float py, int period, uint32_t seed) {
-    float s = 0.f, w = 1.f;
-    for (int o = 0; o < 5; o++) {
-        s = s + w * value2(px, py, period << o, seed + (uint32_t)o);
-        w = w * 0.5f;
-    }
-    return s * (1.0f / 1.9375f);
+// Value noise; at(x, y) gives the lattice points' values.
+template <class At>
+__device__ __forceinline__ float value2(float px, float py, int period, const At& at) {
+    const float qx = px * (float)period, qy = py * (float)period;
+    const float fx = floorf(qx), fy = floorf(qy);
+    const float tx = qx - fx, ty = qy - fy;
+    const int ix = (int)fx, iy = (int)fy;
+    const float sx = (tx * tx) * (3.0f - 2.0f * tx), sy = (ty * ty) * (3.0f - 2.0f * ty);
+    return lerp_(lerp_(at(ix, iy), at(ix + 1, iy), sx), lerp_(at(ix, iy + 1), at(ix + 1, iy + 1), sx), sy);
 }
 
 __device__ __forceinline__ uint32_t q8(float v) {
@@ -393,22 +398,16 @@ __device__ __forceinline__ uint32_t q8(float v) {
 __device__ __forceinline__ uint32_t half_bits(float v) { return (uint32_t)__half_as_ushort(__float2half_rn(v)); }
 
 // Round-to-nearest-even FP8 e4m3 (OCP: bias 7, max finite 448, no infinities) of a value >= 0.
-__device__ __forceinline__ uint32_t fp8_e4m3(float v) {
-    if (!(v > 0.0f)) return 0u;
-    if (v >= 448.0f) return 0x7Eu;
-    uint32_t u = __float_as_uint(v);
-    int e = (int)((u >> 23) & 0xff) - 127;
-    if (e < -6) {  // subnormal: multiples of 2^-9
-        float q = rintf(v * 512.0f);
-        return (uint32_t)q;  // q in [0, 8]; 8 encodes the smallest normal
-    }
-    uint32_t mant = u & 0x7fffffu;
-    uint32_t keep = mant >> 20, rest = mant & 0xfffffu;
-    if (rest > 0x80000u || (rest == 0x80000u && (keep & 1u))) keep++;
-    uint32_t ee = (uint32_t)(e + 7);
-    if (keep == 8u) { keep = 0u; ee++; }
-    uint32_t r = (ee << 3) | keep;
-    return r > 0x7Eu ? 0x7Eu : r;
+// Two values in the low or high half of `r`: the conversion rounds to nearest even, subnormals included. (Compared
+// with the rounding written out, over every float: equal.)
+template <bool HIGH>
+__device__ __forceinline__ uint32_t fp8_pair(float a, float b, uint32_t r) {
+    a = fminf(fmaxf(a, 0.0f), 448.0f);  // NaN: 0
+    b = fminf(fmaxf(b, 0.0f), 448.0f);
+    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, (int)r, HIGH);
+}
+__device__ __forceinline__ uint32_t fp8x4(float a, float b, float c, float d) {
+    return fp8_pair<true>(c, d, fp8_pair<false>(a, b, 0u));
 }
 
 struct GenArgs {
@@ -452,10 +451,7 @@ struct StageMeta {
 // The low-res texel's 32-bit word (RGBA8 or FP8 x 4).
 __device__ __forceinline__ uint32_t encode_low_res(const GenArgs& a, const float v[4]) {
     if (a.fmt == MM_FMT_RGBA8) return q8(v[0]) | (q8(v[1]) << 8) | (q8(v[2]) << 16) | (q8(v[3]) << 24);
-    uint32_t r = 0;  // MM_FMT_FP8X4
-#pragma unroll 1
-    for (int k = 0; k < 4; k++) r |= fp8_e4m3((k < 2 ? (k == 0 ? v[0] : v[1]) : (k == 2 ? v[2] : v[3])) * a.inv_scale[k]) << (8 * k);
-    return r;
+    return fp8x4(v[0] * a.inv_scale[0], v[1] * a.inv_scale[1], v[2] * a.inv_scale[2], v[3] * a.inv_scale[3]);  // MM_FMT_FP8X4
 }
 
 __device__ __forceinline__ void store_hi_res(const GenArgs& a, long i, const float v[3]) {
@@ -498,14 +494,11 @@ inline long box_bound(int b, int dim, int cells, int pad) { return ((long)(b - 1
 // 85, 32^3 hi-res 20 -> 15. Vector operations bound it (27 distances, 9 operations each, at each Worley level).
 // Texels whose coordinate is below the apron width are also written to the apron copy (x + dim, ...).
 template <bool HI>
-__global__ __launch_bounds__(256) void volume_brick_kernel(GenArgs a, int cap) {
-    extern __shared__ float4 cells[];
+__device__ __forceinline__ void volume_brick(const GenArgs& a, int block, int cap, float4* cells, StageMeta* meta) {
     constexpr int kFirstWorley = HI ? 0 : 4;
-    __shared__ StageMeta meta[4];
     const int tid = threadIdx.x;
     const int nbx = (a.dim + kBrickX - 1) / kBrickX, nby = (a.dim + kBrickY - 1) / kBrickY;
-    const int x0 = (int)(blockIdx.x % nbx) * kBrickX, y0 = (int)((blockIdx.x / nbx) % nby) * kBrickY;
-    const int z0 = (int)(blockIdx.x / (nbx * nby)) * kBrickZ;
+    const int x0 = (block % nbx) * kBrickX, y0 = ((block / nbx) % nby) * kBrickY, z0 = block / (nbx * nby) * kBrickZ;
     const int x1 = min(x0 + kBrickX, a.dim) - 1, y1 = min(y0 + kBrickY, a.dim) - 1, z1 = min(z0 + kBrickZ, a.dim) - 1;
     const float inv = 1.0f / (float)(2 * a.dim);
     auto level_cells = [](int l) { return HI ? hi_level_cells(l) : low_level_cells(l); };
@@ -706,8 +699,7 @@ __device__ __forceinline__ void worley128(const float4* cells, const float (&px)
     }
 #pragma unroll
     for (int t = 0; t < k128T; t++) {
-        const float d = sqrt_rn(best[t]);
-        out[t] = 1.0f - (d < 1.0f ? d : 1.0f);
+        out[t] = inverted(best[t]);
     }
     __builtin_amdgcn_sched_barrier(0);  // one level's reads in flight at a time: the levels together would spill
 }
@@ -769,10 +761,9 @@ __device__ __forceinline__ void perlin_fbm128(const float4* cells, const float (
     if constexpr (L < 3) perlin_fbm128<L + 1>(cells, px, py, pz, x0, y0, z0, w * 0.5f, s);
 }
 
-__global__ __launch_bounds__(256, 4) void low_res_128_kernel(GenArgs a) {
-    __shared__ float4 cells[k128LdsCells()];
+__device__ __forceinline__ void low_res_128(const GenArgs& a, int b, float4* cells) {
     constexpr int dim = 128, nbx = dim / k128X, nby = dim / k128Y;
-    const int b = (int)blockIdx.x, tid = (int)threadIdx.x;
+    const int tid = (int)threadIdx.x;
     const int x0 = (b % nbx) * k128X, y0 = (b / nbx % nby) * k128Y, z0 = b / (nbx * nby) * k128Z;
     stage128<0>(cells, a.seed, x0, y0, z0);
     __syncthreads();
@@ -804,25 +795,102 @@ __global__ __launch_bounds__(256, 4) void low_res_128_kernel(GenArgs a) {
         }
 }
 
-__global__ __launch_bounds__(256) void weather_kernel(GenArgs a) {
-    const int sd = a.dim + a.apron;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= sd * sd) return;
-    const int x = (i % sd) % a.dim, y = (i / sd) % a.dim;
+// A block takes 16 x 16 logical texels. The lattice values they touch are hashed once into LDS, level by level
+// (three FBMs of five octaves), while they fit; the others hash in place (small maps at high frequencies). 60
+// hashes a texel of the 512^2 map were 14.6 us of vector operations, now 10.3 alone.
+constexpr int kWeatherTile = 16, kWeatherLevels = 15, kWeatherCap = 4096;
+__device__ __forceinline__ int weather_period(int l) { return (l < 5 ? 4 : 8) << (l % 5); }
+__device__ __forceinline__ uint32_t weather_seed(uint32_t seed, int l) {
+    return layer_seed(seed, 11 + (uint32_t)l / 5) + (uint32_t)l % 5;
+}
+__device__ __forceinline__ void weather_tile(const GenArgs& a, int block, float* values, StageMeta* meta) {
+    const int tid = threadIdx.x, tiles = (a.dim + kWeatherTile - 1) / kWeatherTile;
+    const int x0 = block % tiles * kWeatherTile, y0 = block / tiles * kWeatherTile;
+    const int x1 = min(x0 + kWeatherTile, a.dim) - 1, y1 = min(y0 + kWeatherTile, a.dim) - 1;
     const float inv = 1.0f / (float)(2 * a.dim);
-    float px = (float)(2 * x + 1) * inv, py = (float)(2 * y + 1) * inv;
-    float va = value_fbm(px, py, 4, layer_seed(a.seed, 11));
-    float vb = value_fbm(px, py, 8, layer_seed(a.seed, 12));
-    float vc = value_fbm(px, py, 8, layer_seed(a.seed, 13));
+    if (tid < kWeatherLevels) {
+        StageMeta m{};
+        axis_span(x0, x1, inv, weather_period(tid), 0, m.bx, m.nx);
+        axis_span(y0, y1, inv, weather_period(tid), 0, m.by, m.ny);
+        meta[tid] = m;
+    }
+    __syncthreads();
+    int off = 0;
+    for (int l = 0; l < kWeatherLevels; l++) {
+        const StageMeta m = meta[l];
+        const int cnt = m.nx * m.ny;
+        const bool fits = cnt <= 2 * kWeatherTile * kWeatherTile && off + cnt <= kWeatherCap;  // uniform across the block
+        if (tid == 0) meta[l].off = fits ? off : -1;
+        if (!fits) continue;
+        if (l % 4 == tid / 64) {  // a wave per level, four at a time
+            const float rx = 1.0f / (float)m.nx;  // e / nx as in volume_brick
+            for (int e = tid & 63; e < cnt; e += 64) {
+                const int jy = (int)(((float)e + 0.5f) * rx);
+                values[off + e] = value_at(m.bx + (e - jy * m.nx), m.by + jy, weather_period(l), weather_seed(a.seed, l));
+            }
+        }
+        off += cnt;
+    }
+    __syncthreads();
+    const int x = x0 + tid % kWeatherTile, y = y0 + tid / kWeatherTile;
+    if (x > x1 || y > y1) return;
+    const float px = (float)(2 * x + 1) * inv, py = (float)(2 * y + 1) * inv;
+    float f[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        float s = 0.f, w = 1.f;
+#pragma unroll 1
+        for (int l = 5 * k; l < 5 * k + 5; l++) {
+            const int period = weather_period(l);
+            const StageMeta m = meta[l];
+            const float v = m.off >= 0
+                ? value2(px, py, period, [&](int ix, int iy) { return values[m.off + (iy - m.by) * m.nx + (ix - m.bx)]; })
+                : value2(px, py, period, [&](int ix, int iy) { return value_at(ix, iy, period, weather_seed(a.seed, l)); });
+            s = s + w * v;
+            w = w * 0.5f;
+        }
+        f[k] = s * (1.0f / 1.9375f);
+    }
+    const float va = f[0], vb = f[1], vc = f[2];
     float r = 0.5f + 2.0f * (va - 0.5f);
     float R = clamp01(r + (a.coverage - 0.5f));
     float G = clamp01(0.5f + 1.5f * ((0.5f * va + 0.5f * vc) - 0.5f));
     float B = clamp01(0.5f + 2.5f * (vb - 0.5f));
-    if (a.fmt == MM_FMT_RGBA8) {
-        reinterpret_cast<uint32_t*>(a.dst)[i] = q8(R) | (q8(G) << 8) | (q8(B) << 16) | (255u << 24);
-    } else {  // MM_FMT_RG8: (coverage, type)
-        reinterpret_cast<uint16_t*>(a.dst)[i] = (uint16_t)(q8(R) | (q8(B) << 8));
-    }
+    const int sd = a.dim + a.apron;
+    for (int ys = y; ys < sd; ys += a.dim)
+        for (int xs = x; xs < sd; xs += a.dim) {
+            const long i = (long)ys * sd + xs;
+            if (a.fmt == MM_FMT_RGBA8) {
+                reinterpret_cast<uint32_t*>(a.dst)[i] = q8(R) | (q8(G) << 8) | (q8(B) << 16) | (255u << 24);
+            } else {  // MM_FMT_RG8: (coverage, type)
+                reinterpret_cast<uint16_t*>(a.dst)[i] = (uint16_t)(q8(R) | (q8(B) << 8));
+            }
+        }
+}
+
+// Every generator in one launch (the curl map's table before it, its store after it): the curl field's blocks, the
+// hi-res volume's, the weather map's, then the low-res volume's; any of them may be absent. The small maps'
+// latency hides behind the volume. On a stream beside the volume's they waited for slots among its blocks, and
+// the fork and the join cost 5 and 16 us: all four maps at 128^3 159 us, in one launch 143.
+struct Grids {
+    CurlArgs curl;
+    GenArgs hi, weather, low;
+    int curlBlocks, hiBlocks, weatherBlocks;  // the low-res volume takes the rest
+    int hiCap, lowCap;
+};
+template <bool LOW128>
+__global__ __launch_bounds__(256, LOW128 ? 4 : 1) void maps_kernel(Grids g) {
+    extern __shared__ float4 cells[];
+    __shared__ StageMeta meta[kWeatherLevels];
+    int b = (int)blockIdx.x;
+    if (b < g.curlBlocks) return curl_field(g.curl, b, reinterpret_cast<float*>(cells));
+    b -= g.curlBlocks;
+    if (b < g.hiBlocks) return volume_brick<true>(g.hi, b, g.hiCap, cells, meta);
+    b -= g.hiBlocks;
+    if (b < g.weatherBlocks) return weather_tile(g.weather, b, reinterpret_cast<float*>(cells), meta);
+    b -= g.weatherBlocks;
+    if constexpr (LOW128) low_res_128(g.low, b, cells);
+    else volume_brick<false>(g.low, b, g.lowCap, cells, meta);
 }
 
 // ------------------------------------------------------------------ repacking of RGBA8 linear textures
@@ -852,10 +920,9 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
             break;
         }
         case MM_FMT_FP8X4: {
-            const uint32_t c[4] = {c0, c1, c2, c3};
-            uint32_t r = 0;
-            for (int k = 0; k < 4; k++) r |= fp8_e4m3(((float)c[k] / 255.0f) * a.inv_scale[k]) << (8 * k);
-            reinterpret_cast<uint32_t*>(a.dst)[i] = r;
+            reinterpret_cast<uint32_t*>(a.dst)[i] =
+                fp8x4(((float)c0 / 255.0f) * a.inv_scale[0], ((float)c1 / 255.0f) * a.inv_scale[1],
+                      ((float)c2 / 255.0f) * a.inv_scale[2], ((float)c3 / 255.0f) * a.inv_scale[3]);
             break;
         }
     }
@@ -863,11 +930,10 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + 255) / 256); }
 
-// volume_brick_kernel over every brick, with the LDS its staged levels can need (any brick's boxes are within
-// the bound, so what fits it on the host fits it in the kernel).
+// The cells a brick of the volume stages at most (any brick's boxes are within the bound, so what fits it on the
+// host fits it in the kernel): the largest layer's; a larger level may still be staged in what others leave.
 template <bool HI>
-void launch_bricks(const GenArgs& a, hipStream_t s) {
-    // the most cells a layer's levels can take together; a larger level may still be staged in what others leave
+int stage_cap(const GenArgs& a) {
     long cap = 0;
     for (int l0 = 0; l0 < (HI ? kHiLevels : kLowLevels); l0 += HI || l0 ? 3 : 4) {
         long layer = 0;
@@ -877,11 +943,10 @@ void launch_bricks(const GenArgs& a, hipStream_t s) {
         }
         cap = std::max(cap, layer);
     }
-    cap = std::min<long>(cap, kStageCap);
-    const long bricks = (long)((a.dim + kBrickX - 1) / kBrickX) * ((a.dim + kBrickY - 1) / kBrickY) *
-                        ((a.dim + kBrickZ - 1) / kBrickZ);
-    hipLaunchKernelGGL(volume_brick_kernel<HI>, dim3((unsigned)bricks), dim3(256), (size_t)cap * sizeof(float4), s, a,
-                       (int)cap);
+    return (int)std::min<long>(cap, kStageCap);
+}
+inline long brick_count(const GenArgs& a) {
+    return (long)((a.dim + kBrickX - 1) / kBrickX) * ((a.dim + kBrickY - 1) / kBrickY) * ((a.dim + kBrickZ - 1) / kBrickZ);
 }
 
 }  // namespace
@@ -932,9 +997,7 @@ int static_scratch(void** ptr) {
 }
 
 namespace {
-// A second stream for work that runs beside the caller's (the curl chain's small grids, the hi-res
-// volume and the weather map beside the low-res volume; the reprojection beside a phase march):
-// forked from the caller's stream and joined back into it with events, so a call stays ordered on
+// A second stream for work that runs beside the caller's (the reprojection beside a phase march): forked from the caller's stream and joined back into it with events, so a call stays ordered on
 // that stream and can be captured into a graph. There is one side stream per (device, caller
 // stream): a side stream joins whatever capture its caller's stream is in and stays in it until that
 // capture ends, so work forked from another caller stream must never reach it. Created on first use
@@ -1004,55 +1067,53 @@ int side_join(hipStream_t main, hipStream_t side) {
     return MM_OK;
 }
 
-int launch_generate(const mm_noise_params* p, const mm_noise_set* out, void* workspace, void* stream,
-                    bool allow_side) {
-    hipStream_t main = (hipStream_t)stream;
-    const uint32_t side_work = p->what & (MM_GEN_CURL | MM_GEN_HI_RES | MM_GEN_WEATHER);
-    std::unique_lock<std::mutex> lock;
-    hipStream_t side = nullptr;
-    if (allow_side && (p->what & MM_GEN_LOW_RES) && side_work) {
-        lock = side_lock();
-        side = side_fork(main);
+int launch_generate(const mm_noise_params* p, const mm_noise_set* out, void* workspace, void* stream) {
+    hipStream_t s = (hipStream_t)stream;
+    auto args = [&](const mm_texture& t, uint32_t seed) {
+        return GenArgs{(uint8_t*)t.data, t.width, t.layout == MM_LAYOUT_APRON ? 1 : 0, t.format, seed, p->coverage, {1, 1, 1, 1}};
+    };
+    Grids g{};
+    unsigned blocks = 0;
+    size_t lds = 0;
+    const bool low128 = (p->what & MM_GEN_LOW_RES) && out->low_res.width == 128;
+    if (p->what & MM_GEN_LOW_RES) {
+        g.low = args(out->low_res, p->seed);
+        if (g.low.fmt == MM_FMT_FP8X4)
+            for (int k = 0; k < 4; k++) g.low.inv_scale[k] = 1.0f / out->low_res.scale[k];
+        g.lowCap = stage_cap<false>(g.low);
+        blocks += low128 ? 128 / k128X * (128 / k128Y) * (128 / k128Z) : (unsigned)brick_count(g.low);
+        lds = sizeof(float4) * (low128 ? (size_t)k128LdsCells() : (size_t)g.lowCap);
     }
-    hipStream_t s = side ? side : main;
     if (p->what & MM_GEN_CURL) {
-        const mm_texture& t = out->curl;
         uint8_t* ws = (uint8_t*)workspace;
-        uint8_t* table = ws;
-        uint32_t* mmx = (uint32_t*)(ws + 20480);
-        float* field = (float*)(ws + 20480 + 256);
-        const int dim = t.width;
-        hipLaunchKernelGGL(curl_table_kernel, dim3(blocks_for(kLat * kLat * kLat)), dim3(256), 0, s, table, mmx);
-        hipLaunchKernelGGL(curl_field_kernel, dim3((unsigned)((dim * dim + kCurlTexels - 1) / kCurlTexels)),
-                           dim3(6 * kCurlTexels), 0, s, table, dim, field, mmx);
-        const int apron = t.layout == MM_LAYOUT_APRON ? 1 : 0;
-        const long n = (long)(dim + apron) * (dim + apron);
-        hipLaunchKernelGGL(curl_store_kernel, dim3(blocks_for(n)), dim3(256), 0, s, field, mmx, dim, apron, t.format,
-                           (uint8_t*)t.data);
-    }
-    if (p->what & MM_GEN_HI_RES) {
-        const mm_texture& t = out->hi_res;
-        GenArgs a{(uint8_t*)t.data, t.width, t.layout == MM_LAYOUT_APRON ? 1 : 0, t.format, p->seed, 0.f, {1, 1, 1, 1}};
-        launch_bricks<true>(a, s);
+        const int dim = out->curl.width;
+        g.curl = CurlArgs{ws, (uint32_t*)(ws + 20480), (float*)(ws + 20480 + 256), dim};
+        blocks += g.curlBlocks = (dim * dim + kCurlTexels - 1) / kCurlTexels;
+        lds = std::max(lds, sizeof(float) * 6 * kCurlTexels);
+        hipLaunchKernelGGL(curl_table_kernel, dim3(blocks_for(kLat * kLat * kLat)), dim3(256), 0, s, g.curl.table, g.curl.mm);
     }
     if (p->what & MM_GEN_WEATHER) {
-        const mm_texture& t = out->weather;
-        GenArgs a{(uint8_t*)t.data, t.width, t.layout == MM_LAYOUT_APRON ? 1 : 0, t.format, p->weather_seed, p->coverage,
-                  {1, 1, 1, 1}};
-        const long sd = t.width + a.apron;
-        hipLaunchKernelGGL(weather_kernel, dim3(blocks_for(sd * sd)), dim3(256), 0, s, a);
+        g.weather = args(out->weather, p->weather_seed);
+        const int tiles = (g.weather.dim + kWeatherTile - 1) / kWeatherTile;
+        blocks += g.weatherBlocks = tiles * tiles;
+        lds = std::max(lds, sizeof(float) * kWeatherCap);
     }
-    if (p->what & MM_GEN_LOW_RES) {
-        const mm_texture& t = out->low_res;
-        GenArgs a{(uint8_t*)t.data, t.width, t.layout == MM_LAYOUT_APRON ? 1 : 0, t.format, p->seed, 0.f, {1, 1, 1, 1}};
-        if (t.format == MM_FMT_FP8X4)
-            for (int k = 0; k < 4; k++) a.inv_scale[k] = 1.0f / t.scale[k];
-        if (t.width == 128) hipLaunchKernelGGL(low_res_128_kernel, dim3(128 / k128X * (128 / k128Y) * (128 / k128Z)), dim3(256), 0, main, a);
-        else launch_bricks<false>(a, main);
+    if (p->what & MM_GEN_HI_RES) {
+        g.hi = args(out->hi_res, p->seed);
+        g.hiCap = stage_cap<true>(g.hi);
+        // beside the low-res volume no more than its blocks' LDS: more would leave fewer of them on a CU (a 9^3
+        // hi-res volume's levels of 64 cells would take 54 KB; a 97^3 low-res one needs 30: 196 us against 160)
+        if (p->what & MM_GEN_LOW_RES) g.hiCap = std::min(g.hiCap, (int)(lds / sizeof(float4)));
+        blocks += g.hiBlocks = (int)brick_count(g.hi);
+        lds = std::max(lds, sizeof(float4) * (size_t)g.hiCap);
     }
-    if (side) {
-        const int e = side_join(main, side);
-        if (e) return e;
+    if (blocks) hipLaunchKernelGGL(low128 ? maps_kernel<true> : maps_kernel<false>, dim3(blocks), dim3(256), lds, s, g);
+    if (p->what & MM_GEN_CURL) {
+        const mm_texture& t = out->curl;
+        const int dim = t.width, apron = t.layout == MM_LAYOUT_APRON ? 1 : 0;
+        const long n = (long)(dim + apron) * (dim + apron);
+        hipLaunchKernelGGL(curl_store_kernel, dim3(blocks_for(n)), dim3(256), 0, s, g.curl.field, g.curl.mm, dim, apron,
+                           t.format, (uint8_t*)t.data);
     }
     return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
 }
