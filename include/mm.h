@@ -284,7 +284,7 @@ int mm_march_clouds_state(const mm_camera_ubo* camera, const mm_sun_ubo* sun, co
  * trips). A schedule records each tile's cost (the most loop trips any of its rays took) in one
  * launch; the next launch of the same shape (tile count, tiles per row, marched grid, kernel shape)
  * first orders its tiles longest first from those costs (a counting sort over log-scale cost
- * buckets, three small launches on the stream) and then marches in that order, recording the new
+ * buckets, two small launches on the stream) and then marches in that order, recording the new
  * costs. Costs are indexed by the tile's
  * place in the image, so they stay valid as the camera moves; a launch of another shape marches in
  * the default order and starts a new record. The image does not depend on the order, bit for bit:
@@ -412,7 +412,7 @@ int mm_load_volume_rgba8(const char* prefix, int32_t depth, uint8_t* rgba, size_
  * wave each), handed to the CUs by the hardware dispatcher as slots free up. Views share the curl
  * and noise volumes and bring their own uniforms, weather map and output image. Each view's image is identical to mm_march_clouds of that view with the same
  * params. A plan holds the per-view constants in device memory; mm_march_views enqueues the march
- * (after the plan's first launch, preceded by three small launches that order all views' tiles
+ * (after the plan's first launch, preceded by two small launches that order all views' tiles
  * longest first by the previous launch's tile costs; the images do not depend on the order) with
  * no allocation, no host transfer and no memset, so it can be captured into a HIP graph and
  * replayed (a capture of the plan's first launch keeps the launch order). */

@@ -1826,10 +1826,11 @@ int launch_t(const MarchConsts& c, const MarchTextures& t, float* out, unsigned 
 
 // ---------------------------------------------------------------- tile schedule
 // Longest-first order of the physical tiles from their costs in the previous launch of the same shape,
-// in three launches over blocks of kOrderChunk tiles: (1) each block's histogram of cost buckets
-// added into the record's per-bucket counts; (2) one workgroup turns the counts into each bucket's
-// first slot, from the largest bucket down; (3) each block reserves a run of slots per bucket with one
-// global atomic and hands them to its tiles with LDS atomics. Every tile gets exactly one slot of
+// in two launches over blocks of kOrderChunk tiles: (1) each block's histogram of cost buckets
+// added into the record's per-bucket counts; (2) each block turns the counts into every bucket's
+// first slot, from the largest bucket down, reserves a run of slots per bucket with one
+// global atomic and hands them to its tiles with LDS atomics. (With the first slots from a
+// launch of one workgroup between the two, scheduled frames took 1-3 us more: 256 x 256 135 us against 132.) Every tile gets exactly one slot of
 // [0, n), so the result is a permutation; the order within a bucket is whatever the atomics give
 // (the image does not depend on the order). The march that follows clears the counts (its block 0)
 // and records the new costs.
@@ -1877,6 +1878,7 @@ __global__ __launch_bounds__(kOrderBlock) void order_count_kernel(unsigned* __re
     unsigned bk[kOrderPer];
     order_block_counts(sched + mm::kSchedHeader, n, cnt, bk);
     for (int b = threadIdx.x; b < kOrderBuckets; b += kOrderBlock) {
+        if (blockIdx.x == 0) sched[mm::kSchedCursor + b] = 0u;  // for the placing launch
         unsigned s = 0;
 #pragma unroll
         for (int r = 0; r < kOrderCopies; r++) s += cnt[b * kOrderCopies + r];
@@ -1884,28 +1886,40 @@ __global__ __launch_bounds__(kOrderBlock) void order_count_kernel(unsigned* __re
     }
 }
 
-// One workgroup of kOrderBuckets threads: thread t takes bucket kOrderBuckets - 1 - t; an inclusive
-// wave scan of the counts, then the wave totals, give each bucket's first slot.
-__global__ __launch_bounds__(kOrderBuckets) void order_scan_kernel(unsigned* __restrict__ sched) {
-    __shared__ unsigned part[kOrderBuckets / 64];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, b = kOrderBuckets - 1 - t;
-    const unsigned mine = sched[mm::kSchedCount + b];
-    unsigned incl = mine;
+// Each bucket's first slot: thread t takes the kOrderPart buckets from kOrderBuckets - 1 - kOrderPart t down; an
+// inclusive wave scan of their sums, then the wave totals.
+constexpr int kOrderPart = kOrderBuckets / kOrderBlock;
+static_assert(kOrderPart * kOrderBlock == kOrderBuckets, "buckets per thread");
+__device__ __forceinline__ void order_starts(const unsigned* __restrict__ counts, unsigned* start, unsigned* part) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, top = kOrderBuckets - 1 - kOrderPart * t;
+    unsigned mine[kOrderPart], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kOrderPart; k++) {
+        mine[k] = counts[top - k];
+        sum += mine[k];
+    }
+    unsigned incl = sum;
     for (int o = 1; o < 64; o <<= 1) {
         const unsigned v = (unsigned)__shfl_up((int)incl, o);
         if (lane >= o) incl += v;
     }
     if (lane == 63) part[wave] = incl;
     __syncthreads();
-    unsigned before = 0;
-    for (int w = 0; w < wave; w++) before += part[w];
-    sched[mm::kSchedCursor + b] = before + incl - mine;
+    unsigned at = incl - sum;
+    for (int w = 0; w < wave; w++) at += part[w];
+#pragma unroll
+    for (int k = 0; k < kOrderPart; k++) {
+        start[top - k] = at;
+        at += mine[k];
+    }
+    __syncthreads();
 }
 
 __global__ __launch_bounds__(kOrderBlock) void order_place_kernel(unsigned* __restrict__ sched, int n,
                                                                    int* __restrict__ order) {
-    __shared__ unsigned cnt[kOrderBuckets * kOrderCopies];
+    __shared__ unsigned cnt[kOrderBuckets * kOrderCopies], start[kOrderBuckets], part[kOrderBlock / 64];
     unsigned bk[kOrderPer];
+    order_starts(sched + mm::kSchedCount, start, part);
     order_block_counts(sched + mm::kSchedHeader, n, cnt, bk);
     // the block's run of slots per bucket, split among the copies
     for (int b = threadIdx.x; b < kOrderBuckets; b += kOrderBlock) {
@@ -1915,7 +1929,7 @@ __global__ __launch_bounds__(kOrderBlock) void order_place_kernel(unsigned* __re
             loc[r] = s;
             s += cnt[b * kOrderCopies + r];
         }
-        const unsigned first = s ? atomicAdd(&sched[mm::kSchedCursor + b], s) : 0u;
+        const unsigned first = s ? start[b] + atomicAdd(&sched[mm::kSchedCursor + b], s) : 0u;
 #pragma unroll
         for (int r = 0; r < kOrderCopies; r++) cnt[b * kOrderCopies + r] = first + loc[r];
     }
@@ -1980,8 +1994,6 @@ int launch_tile_order(unsigned* sched, int n, int* order, void* stream) {
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid((unsigned)((n + kOrderChunk - 1) / kOrderChunk));
     hipLaunchKernelGGL(order_count_kernel, grid, dim3(kOrderBlock), 0, s, sched, n);
-    if (hipGetLastError() != hipSuccess) return MM_E_DEVICE;
-    hipLaunchKernelGGL(order_scan_kernel, dim3(1), dim3(kOrderBuckets), 0, s, sched);
     if (hipGetLastError() != hipSuccess) return MM_E_DEVICE;
     hipLaunchKernelGGL(order_place_kernel, grid, dim3(kOrderBlock), 0, s, sched, n, order);
     return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;

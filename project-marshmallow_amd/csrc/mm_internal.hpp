@@ -165,7 +165,7 @@ const uint4* surrogate_infer_frags(const void* model);  // FP16 inference fragme
 int launch_march(int fset, const MarchConsts& c, const MarchTextures& t, float* out, unsigned long long* counts,
                  void* stream);
 // order <- the n physical tiles of a schedule record sorted by cost, largest first (bucketed: 1024 cost
-// buckets), in three launches on `stream`. The record's counts must be clear (every scheduled march
+// buckets), in two launches on `stream`. The record's counts must be clear (every scheduled march
 // clears them for the next order).
 int launch_tile_order(unsigned* sched, int n, int* order, void* stream);
 
