@@ -1601,8 +1601,14 @@ __global__ __launch_bounds__(64) void march_rp_kernel(const MarchConsts c, const
 // inputs) already holds a CU to 22 waves, 5 per SIMD, so the cap is 5: at 6 the MLP spills to
 // scratch for no extra wave (1080p, every cone replaced, two lanes per ray: 4 / 5 / 6 waves
 // 2.27 / 2.15 / 2.22 ms).
+// The counting instances carry up to 47 more spilled registers at that cap, and for some of them the compiler
+// put the spills of values that are live in every lane before the s_or that ends the features' `if (lane < nb)`:
+// lanes past a short batch came back with stale values and the image was wrong. At 3 waves (up to 168
+// registers) they spill none; tests/test_spill_masks.py looks for such spills in every kernel built.
+template <bool COUNT>
+constexpr int kSurrogateWaves = COUNT ? 3 : MM_SURROGATE_WAVES_PER_EU;
 template <int FSET, bool COUNT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MM_SURROGATE_WAVES_PER_EU)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSurrogateWaves<COUNT>)))
 void march_surrogate_kernel(const MarchConsts c, const MarchTextures tx, float* __restrict__ out,
                             unsigned long long* __restrict__ counts) {
     const int tile = block_tile(c);
@@ -1612,7 +1618,7 @@ void march_surrogate_kernel(const MarchConsts c, const MarchTextures tx, float* 
 
 // The surrogate-lit march with two lanes per ray (the plain march's default shape for full frames).
 template <int FSET, bool COUNT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MM_SURROGATE_WAVES_PER_EU)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSurrogateWaves<COUNT>)))
 void march_rp_surrogate_kernel(const MarchConsts c, const MarchTextures tx, float* __restrict__ out,
                                unsigned long long* __restrict__ counts) {
     const int tile = block_tile(c);
@@ -1743,7 +1749,7 @@ void march_views_kernel(const ViewDesc* __restrict__ views, int nViews, const Ma
 }
 
 template <int FSET, bool COUNT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MM_SURROGATE_WAVES_PER_EU)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSurrogateWaves<COUNT>)))
 void march_views_surrogate_kernel(const ViewDesc* __restrict__ views, int nViews, const MarchTextures tx, int total,
                                   unsigned long long* __restrict__ counts, const int* __restrict__ order,
                                   unsigned* __restrict__ sched) {
