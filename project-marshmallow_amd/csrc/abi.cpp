@@ -574,13 +574,16 @@ static void schedule_key(const mm::MarchConsts& c, int key[6]) {
 
 // Hooks a schedule into a built launch: the march records each tile's cost, and when the schedule
 // holds the costs of a launch of the same shape, a longest-first order built from them on the stream
-// first. The lock-step kernel takes no schedule (it keeps the shader's structure).
+// first. The lock-step kernel takes no schedule (it keeps the shader's structure): it neither follows an
+// order nor clears the record's counts, which would then add up in the next order and lose tiles. The float
+// sampler's plain cones run on it too; the record keeps the costs it had.
 static int use_schedule(mm::MarchConsts& c, mm_march_schedule* sched, void* stream) {
     if (!sched || (c.flags & MM_MARCH_NO_BATCH)) return MM_OK;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return MM_E_DEVICE;
     if (dev != sched->device) return MM_E_PARAM;
     if (c.tiles > sched->capacity) return MM_E_SIZE;
+    if (c.subtexelBits == 0 && c.coneMode == MM_CONE_PLAIN) return MM_OK;
     int key[6];
     schedule_key(c, key);
     if (sched->history && memcmp(key, sched->key, sizeof(key)) == 0) {
