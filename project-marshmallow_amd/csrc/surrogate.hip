@@ -1,5 +1,5 @@
 // Learned light-cone surrogate: parameter init, feature statistics, BF16 fragment packing, MFMA
-// training step (forward, backward, gradient accumulation), Adam, and batch prediction.
+// training step (forward, backward, gradient accumulation) and Adam.
 //
 // The model predicts, for one light-cone job of the march (comp:441-453), the log sun
 // transmittance o0 = -D (D = density along the light) and an error bound e = softplus(o1) in
@@ -471,22 +471,6 @@ __global__ void zero_kernel(float* p, int n, float* one) {
     if (i == 0 && one) *one = 0.0f;
 }
 
-// Batch inference with the march's FP16 path: 64 samples per wave; out[i] = (o0, softplus(o1)).
-__global__ __launch_bounds__(64) void predict_kernel(const float* __restrict__ x, int n, int stride,
-                                                     const float* __restrict__ params, const float* __restrict__ stats,
-                                                     const uint4* __restrict__ hfrags, float* __restrict__ out) {
-    const int lane = threadIdx.x;
-    const long i = (long)blockIdx.x * 64 + lane;
-    float f[kIn];
-    for (int k = 0; k < kIn; k++) f[k] = i < n ? (x[i * stride + k] - stats[k]) * stats[16 + k] : 0.0f;
-    const long left = (long)n - (long)blockIdx.x * 64;
-    FwdOut o = mlp_infer64_h(hfrags, params + oB4, f, left < 64 ? (int)left : 64);
-    if (i < n) {
-        out[i * 2 + 0] = o.o0;
-        out[i * 2 + 1] = softplus(o.o1);
-    }
-}
-
 inline unsigned blocks(long n, int b) { return (unsigned)((n + b - 1) / b); }
 
 }  // namespace
@@ -557,13 +541,6 @@ int surrogate_gradient(const void* model, const float* samples, int n, int strid
     const unsigned nb = std::min(blocks(n, kTrainRows), (unsigned)kMaxTrainBlocks);
     hipLaunchKernelGGL(train_kernel<true>, dim3(nb), dim3(64 * kTrainWaves), 0, s, samples, n, stride, p.params,
                        p.stats, p.frags, grad_out, loss_out, 0u, nullptr, 0, n, 1.0f / (float)n);
-    return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
-}
-
-int surrogate_predict(const void* model, const float* x, int n, int stride, float* out, void* stream) {
-    ModelPtrs p = ptrs(const_cast<void*>(model));
-    hipLaunchKernelGGL(predict_kernel, dim3(blocks(n, 64)), dim3(64), 0, (hipStream_t)stream, x, n, stride, p.params,
-                       p.stats, p.hfrags, out);
     return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
 }
 
