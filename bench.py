@@ -291,7 +291,8 @@ def lanes_and_tiles(args):
     if args.no_schedule:
         lanes = args.lanes_per_ray or (16 if rays <= 45_000 else 8 if rays <= 400_000 else 2)
     else:
-        lanes = args.lanes_per_ray or (16 if rays <= 45_000 else 8 if rays <= 200_000 else 4 if rays <= 480_000 else 2 if rays <= 1 << 20 else 1)
+        lanes = args.lanes_per_ray or (1 if args.tile_width else 16 if rays <= 45_000 else 8 if rays <= 200_000
+                                       else 4 if rays <= 480_000 else 2 if rays <= 1 << 20 else 1)
     if lanes > 1:
         return lanes, 4 if lanes == 16 else 8
     return 1, args.tile_width or (8 if args.no_schedule else 16)

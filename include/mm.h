@@ -211,14 +211,16 @@ typedef struct mm_march_params {
     float surrogate_threshold;  /* jobs whose weighted error bound is >= this take the plain cone */
     const void* surrogate;      /* device model block of mm_surrogate_bytes() (MM_CONE_SURROGATE);
                                    REF and FAST texture sets only */
-    int32_t tile_width;         /* pixels per wave tile row: 8 (8x8, default when 0), 16 (16x4), 32 (32x2);
-                                   the image does not depend on it */
+    int32_t tile_width;         /* pixels per wave tile row with one lane per ray: 8 (8x8, default when 0),
+                                   16 (16x4), 32 (32x2); a width asked for through a schedule, with
+                                   lanes_per_ray 0, takes one lane per ray; the image does not depend on it */
     int32_t lanes_per_ray;      /* 1, 2, 4 or 8 lanes march one ray, sampling the next trips ahead
                                    and committing them in order (0 = default, by the rays marched:
-                                   16 up to 45 000 of them, 8 for a phase of up to 2^19 rays and a frame of up to 400 000, else
-                                   2; through a schedule 8, 4, 2 and 1 from the smallest frames to
-                                   those over 2^20 rays); plain cones only (the surrogate-lit march
-                                   takes at most 2, other modes 1); the image does not depend on it */
+                                   16 up to 45 000 of them (16 only as a default), 8 for a phase of up to
+                                   2^19 rays and a frame of up to 400 000, else 2; through a schedule 8, 4,
+                                   2 and 1 from the smallest frames to those over 2^20 rays); plain cones
+                                   only (the surrogate-lit march takes at most 2, other modes 1); the image
+                                   does not depend on it */
     int32_t _reserved[6];
 } mm_march_params;
 

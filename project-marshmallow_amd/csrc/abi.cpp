@@ -495,9 +495,13 @@ struct mm_march_schedule {
 // The ray-parallel kernel's tiles: 8 x (8 / lanes) rays, 4 x 1 with 16 lanes.
 static int tile_shift(int lanes) { return lanes == 16 ? 2 : 3; }
 
-// Lanes per ray of a march (params.lanes_per_ray; 0 = by the rays, see kFrameRays8); 1 for the other cone
-// modes and the lock-step kernel. A schedule takes no more lanes than its record holds the tiles of (the
-// one-lane tiles are the fewest). The image does not depend on it.
+// Lanes per ray of a march (params.lanes_per_ray; 0 = by the rays, see kFrameRays8); 1 for the recorder and
+// the lock-step kernel. A schedule takes no more lanes than its record holds the tiles of (the
+// one-lane tiles are the fewest). A tile width asked for through a schedule asks for the one-lane kernel,
+// which alone has it. The float sampler's kernels march 64 rays a wave whatever this says: in the tiles of more
+// lanes most of its blocks hold no ray and end at once, which costs less than one-lane tiles do (us, lanes by the
+// rays / one: one phase of 200 x 200 1401 / 1609, of 760 x 540 1901 / 2155; surrogate-lit 1080p 1502 / 1908).
+// The image does not depend on any of it.
 static int lanes_for(const mm::MarchConsts& c, const mm_march_params* params, int32_t phase,
                      const mm_march_schedule* sched = nullptr) {
     int lpr = params ? params->lanes_per_ray : 0;
@@ -514,6 +518,7 @@ static int lanes_for(const mm::MarchConsts& c, const mm_march_params* params, in
         };
         if (sched)
             while (lpr > (one_phase ? 8 : 1) && tiles(lpr) > sched->capacity) lpr /= 2;
+        if (sched && !one_phase && params && params->tile_width != 0) lpr = 1;
     }
     if (c.flags & MM_MARCH_NO_BATCH) return 1;
     // the surrogate-lit march runs with one or two lanes per ray; the sample recorder with one
