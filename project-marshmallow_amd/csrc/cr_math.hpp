@@ -76,3 +76,20 @@ __device__ __forceinline__ float div_rn_normal(float n, float d) {
     q = __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
     return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
 }
+
+// Two values, as FP8 e4m3 (OCP: bias 7, max finite 448, no infinities), in the low or high half of r: negative
+// values and NaN give 0, the conversion rounds to nearest even, subnormals included. tests/c/cvt_gpu_check.hip
+// compares it with the rounding written out over every float.
+template <bool HIGH>
+__device__ __forceinline__ unsigned fp8_pair(float a, float b, unsigned r) {
+    a = fminf(fmaxf(a, 0.0f), 448.0f);
+    b = fminf(fmaxf(b, 0.0f), 448.0f);
+    return (unsigned)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, (int)r, HIGH);
+}
+
+// floor(v + 0.5), exactly (the addition is not rounded to float), for |v| below 2^31.
+__device__ __forceinline__ int floor_half_up(float v) {
+    int k;
+    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(k) : "v"(v));
+    return k;
+}

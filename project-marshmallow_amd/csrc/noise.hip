@@ -397,15 +397,6 @@ __device__ __forceinline__ uint32_t q8(float v) {
 
 __device__ __forceinline__ uint32_t half_bits(float v) { return (uint32_t)__half_as_ushort(__float2half_rn(v)); }
 
-// Round-to-nearest-even FP8 e4m3 (OCP: bias 7, max finite 448, no infinities) of a value >= 0.
-// Two values in the low or high half of `r`: the conversion rounds to nearest even, subnormals included. (Compared
-// with the rounding written out, over every float: equal.)
-template <bool HIGH>
-__device__ __forceinline__ uint32_t fp8_pair(float a, float b, uint32_t r) {
-    a = fminf(fmaxf(a, 0.0f), 448.0f);  // NaN: 0
-    b = fminf(fmaxf(b, 0.0f), 448.0f);
-    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, (int)r, HIGH);
-}
 __device__ __forceinline__ uint32_t fp8x4(float a, float b, float c, float d) {
     return fp8_pair<true>(c, d, fp8_pair<false>(a, b, 0u));
 }

@@ -46,8 +46,10 @@ __device__ __forceinline__ void axis(float u, int n, int bits, int& i0, int& i1,
 
 // Taps of which every texel exists, weights of 1/256 (about 70 issue cycles against 190 for tap_edge): no clamps,
 // one 8-byte load a row. u (256 n) - 128 is 256 times u n - 0.5 with the same roundings, and k = floor(that + 0.5)
-// holds the texel (k >> 8) and 256 times its weight (k & 255); v_cvt_rpi_i32_f32 is the exact floor(v + 0.5),
-// which differs from adding in float only at 0.5 - 2^-25, no difference from 128.
+// holds the texel (k >> 8) and 256 times its weight (k & 255). The exact floor_half_up is the floor of the sum rounded
+// to float, as the restatement takes it, for every v here: at most 2^22 (256 texels of 16384), where 0.5 is a
+// multiple of the sum's last place, and, as a difference from 128, a multiple of 2^-17, so no v lies so close
+// under 0.5 that the sum would round up to 1 (tests/c/cvt_gpu_check.hip compares the two over all of them).
 struct Map {
     float w256, h256;  // in vector registers: a float instruction with a scalar operand issues at half the rate
     float right, bottom;
@@ -96,8 +98,8 @@ __device__ __forceinline__ float tap_edge(const float* __restrict__ img, const m
     return lerp_r(lerp_r(t00, t01, fx), lerp_r(t10, t11, fx), fy);
 }
 __device__ __forceinline__ void texel(const At& a, int& kx, int& ky, float& fx, float& fy) {
-    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(kx) : "v"(a.x));
-    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(ky) : "v"(a.y));
+    kx = floor_half_up(a.x);
+    ky = floor_half_up(a.y);
     fx = (float)(kx & 255) * (1.0f / 256.0f);
     fy = (float)(ky & 255) * (1.0f / 256.0f);
 }
