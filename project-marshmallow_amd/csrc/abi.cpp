@@ -285,6 +285,11 @@ struct CollectArgs {
 //     230 400: 839 491 269 247 / 573 335 209 247;  518 400: 785 459 420 473 / 622 384 394 506;
 //     921 600: 807 641 712 820 / 681 616 653 872;  1 440 000: 915 964 1087 1268 / 853 913 985 1341
 //   one phase  518 400: 826 600 549 459 / 613 401 475 467;  921 600: 1137 684 855 841 / 875 617 727 874
+// (Past 400 000 rays an unscheduled frame would do better with 4 lanes on both scenes at 409 920, on one at
+// 518 400 and on neither at 921 600; the rule has no such band.)
+// The surrogate-lit march takes 2 lanes where this says 2 or more. Through a schedule, 1 and 2 lanes:
+//   65 536 rays 778 432 / 568 298;  518 400: 914 525 / 650 375;  1 048 320: 960 693 / 724 591;
+//   1 440 000: 997 884 / 773 796
 // 16 lanes pay for both scenes up to 45 000 rays or so, 8 and 16 lanes: 16 384 rays 121 77 / 84 63; one phase
 //   32 400: 140 92 / 104 83;  57 600: 147 111 / 107 120;  65 536: 141 112 / 110 132.
 constexpr long long kRays16 = 45000;

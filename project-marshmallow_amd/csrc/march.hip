@@ -1616,7 +1616,7 @@ void march_surrogate_kernel(const MarchConsts c, const MarchTextures tx, float* 
     march_tile<FSET, COUNT, CONE_SURROGATE>(c, tx, tile, out, counts, CostRec{c.tileSched, tile});
 }
 
-// The surrogate-lit march with two lanes per ray (the plain march's default shape for full frames).
+// The surrogate-lit march with two lanes per ray: its default below 2^20 rays and, unscheduled, at every size.
 template <int FSET, bool COUNT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSurrogateWaves<COUNT>)))
 void march_rp_surrogate_kernel(const MarchConsts c, const MarchTextures tx, float* __restrict__ out,

@@ -36,8 +36,8 @@ struct MarchConsts {
     int width, height, pitch;    // image size used for uv and bounds, row pitch in pixels
     int phase;                   // -1 = all pixels
     int gridW, gridH;            // marched pixel grid
-    int tileShift;                // tiles of (1 << tileShift) x (64 >> tileShift) pixels: 3, 4 or 5
-    int lanesPerRay;              // 1, or 2 / 4 / 8 for the ray-parallel kernel (tiles of 8 x (8 / lanesPerRay) rays)
+    int tileShift;                // tiles of (1 << tileShift) x ((64 / lanesPerRay) >> tileShift) pixels: 3, 4 or 5; 2 with 16 lanes
+    int lanesPerRay;              // 1, or 2 / 4 / 8 / 16 for the ray-parallel kernel (tiles of 8 x (8 / lanesPerRay) rays, 4 x 1 with 16)
     int tilesX, tilesY;           // tiles of the marched grid
     int tiles;                    // tilesX * tilesY: one block per tile
     int rowStart, rowDir;         // launch order of tile rows: logical row r is row (rowStart + rowDir r) mod tilesY

@@ -24,7 +24,9 @@ constexpr size_t offParams = 0, offGrads = kPadP, offM = 2 * kPadP, offV = 3 * k
 constexpr int kPackThreads = (kFrags + kHFrags) * 64;
 
 struct ModelPtrs {
-    float *params, *grads, *m, *v, *stats;  // stats: mean[16], inv_std[16], step, loss_sum, loss_n
+    // grads: nothing reads it (training sums its gradients in buffers of its own); its place keeps the layout of
+    // saved blocks, and zeros make a new block the same bytes every time. stats: mean[16], inv_std[16], step, loss
+    float *params, *grads, *m, *v, *stats;
     uint4* frags;   // BF16 training fragments (kFrags)
     uint4* hfrags;  // FP16 inference fragments (kHFrags)
 };
