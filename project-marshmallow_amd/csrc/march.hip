@@ -1675,7 +1675,8 @@ __global__ __launch_bounds__(64) void cloud_shadow_kernel(const mm::ShadowConsts
     const unsigned i = lane >> split;
     if (i >= (unsigned)c.n) return;
     const int first = (int)(lane & ((1u << split) - 1u));
-    const V3 wc = mk(pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]);
+    const float* pt = pts + (size_t)i * 3;  // 64 bits: 3 i passes 32 from 1.4 G points on
+    const V3 wc = mk(pt[0], pt[1], pt[2]);
     const V3 sunW = ld3(c.sunW);
     const V3 camPos = ld3(c.camPos);
     V3 center = camPos;
