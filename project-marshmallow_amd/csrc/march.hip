@@ -1981,9 +1981,12 @@ namespace mm {
 int launch_shadow(int fset, const ShadowConsts& c, const TexView& weather, const TexView& low, const float* pts,
                   float* out, void* stream) {
     // Few points are bound by a lane's chain of steps, many by their scattered texel reads. us at 1, 2, 8 lanes a
-    // point (256-point blocks of one lane: 14.6 / 15.1 / 15.9 / 25.8 / 686): 20 011 points 12.3 9.6 8.1;
-    // 40 000 13.2 11.6 11.5; 65 536 15.9 15.5 17.2; 100 000 22.9 22.6 24.7; 4 M 685 688 785.
-    int split = c.n <= 32768 ? 3 : c.n <= 65536 ? 1 : 0;
+    // point, apron / linear textures, sun at 60 degrees (256-point blocks of one lane before: 20 011 points 15.6 / 18.2,
+    // 55 000 17.2 / 20.0, 65 536 18.2 / 21.0, 66 000 27.4 / 35.2, 2 M 431 / 549): 20 011 12.9 9.9 9.2 / 15.3 10.9 10.3;
+    // 32 768 13.6 12.0 12.1 / 15.8 13.2 13.9;  33 000 13.8 12.6 12.5 / 16.5 14.4 14.4;  50 000 17.2 16.1 17.6 / 19.8 19.1
+    // 19.1;  55 000 17.7 16.4 18.4 / 20.3 19.5 20.3;  60 000 17.9 18.0 19.9 / 20.3 21.4 21.9;  65 536 18.3 18.4 20.5 /
+    // 20.8 21.9 23.2. With lower suns 2 lanes stay ahead to 65 536.
+    int split = c.n <= 32768 ? 3 : c.n <= 57344 ? 1 : 0;
     while (split > 0 && 1 << (split - 1) >= c.steps) split--;  // no lane without a step
     dim3 grid((unsigned)((((unsigned long long)c.n << split) + 63) / 64)), block(64);
     hipStream_t s = (hipStream_t)stream;
