@@ -154,6 +154,7 @@ int surrogate_fit_stats(void* model, const float* samples, int n, int stride, vo
 int surrogate_train(void* model, const float* samples, int n, int stride, int batch, int steps, float lr,
                     uint32_t seed, float* loss_out, void* stream);
 int surrogate_predict(const void* model, const float* x, int n, int stride, float* out, void* stream);
+int surrogate_predict_few(const void* model, const float* x, int n, int stride, float* out, void* stream);
 int surrogate_load(void* model, const float* params, const float* stats, void* stream);
 int surrogate_gradient(const void* model, const float* samples, int n, int stride, float* grad_out, float* loss_out,
                        void* stream);

@@ -1,39 +1,18 @@
-// Batch prediction of the learned light-cone surrogate: a translation unit of its own, without the flag that keeps
-// the training kernel's MFMA accumulators in ordinary registers. With it this kernel takes 91 registers, all
-// ordinary, and 500 000 rows 36.5 us; without it, accumulators in the accumulator file, 34.4 us.
+// Batch prediction of the learned light-cone surrogate, and the choice of its kernel's form (predict_dev.hpp).
 #include <hip/hip_runtime.h>
-#include "mm_internal.hpp"
-#include "surrogate_dev.hpp"
-
-using namespace surr;
-
-namespace {
-
-// Batch inference with the march's FP16 path: 64 samples per wave; out[i] = (o0, softplus(o1)).
-__global__ __launch_bounds__(64) void predict_kernel(const float* __restrict__ x, int n, int stride,
-                                                     const float* __restrict__ params, const float* __restrict__ stats,
-                                                     const uint4* __restrict__ hfrags, float* __restrict__ out) {
-    const int lane = threadIdx.x;
-    const long i = (long)blockIdx.x * 64 + lane;
-    float f[kIn];
-    for (int k = 0; k < kIn; k++) f[k] = i < n ? (x[i * stride + k] - stats[k]) * stats[16 + k] : 0.0f;
-    const long left = (long)n - (long)blockIdx.x * 64;
-    FwdOut o = mlp_infer64_h(hfrags, params + oB4, f, left < 64 ? (int)left : 64);
-    if (i < n) {
-        out[i * 2 + 0] = o.o0;
-        out[i * 2 + 1] = softplus(o.o1);
-    }
-}
-
-}  // namespace
+#include "predict_dev.hpp"
 
 namespace mm {
 
+// Ordinary registers while their five waves a SIMD (1024 SIMDs, 64 rows a wave: 327 680 rows) take the rows at once
+// or nearly so, the accumulator file beyond. us, ordinary / accumulator file: 1000 rows 5.3 / 6.1, 100 000 7.1 / 7.7,
+// 300 000 20.4 / 23.3, 327 680 22.1 / 24.3, 348 000 24.8 / 24.8; 360 000 25.9 / 25.3, 400 000 28.4 / 27.4, 500 000
+// 34.6 / 32.3, 800 000 50.4 / 51.5, 1 M 61.0 / 61.2, 2 M 112.8 / 111.6, 4 M 233 / 229.
+constexpr int kFewRows = 348000;
+
 int surrogate_predict(const void* model, const float* x, int n, int stride, float* out, void* stream) {
-    const unsigned blocks = (unsigned)(((long)n + 63) / 64);
-    hipLaunchKernelGGL(predict_kernel, dim3(blocks), dim3(64), 0, (hipStream_t)stream, x, n, stride,
-                       surrogate_params(model), surrogate_stats(model), surrogate_infer_frags(model), out);
-    return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
+    return n <= kFewRows ? surrogate_predict_few(model, x, n, stride, out, stream)
+                              : launch_predict(model, x, n, stride, out, stream);
 }
 
 }  // namespace mm

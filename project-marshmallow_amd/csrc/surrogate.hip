@@ -10,6 +10,7 @@
 #include <algorithm>
 #include "mm_internal.hpp"
 #include "surrogate_dev.hpp"
+#include "predict_dev.hpp"
 
 using namespace surr;
 
@@ -544,6 +545,11 @@ int surrogate_gradient(const void* model, const float* samples, int n, int strid
     hipLaunchKernelGGL(train_kernel<true>, dim3(nb), dim3(64 * kTrainWaves), 0, s, samples, n, stride, p.params,
                        p.stats, p.frags, grad_out, loss_out, 0u, nullptr, 0, n, 1.0f / (float)n);
     return hipGetLastError() == hipSuccess ? MM_OK : MM_E_DEVICE;
+}
+
+// Prediction with this file's MFMA form (see predict.hip for when).
+int surrogate_predict_few(const void* model, const float* x, int n, int stride, float* out, void* stream) {
+    return launch_predict(model, x, n, stride, out, stream);
 }
 
 const float* surrogate_params(const void* model) { return ptrs(const_cast<void*>(model)).params; }
